@@ -12,8 +12,7 @@
 //
 // At decode batch sizes the product is bound by reading the weights (V H 2
 // bytes, read once per pass of up to 8 hidden rows); batches that would need
-// more than one such pass take the MFMA tiling further down (one pass per 256
-// rows).
+// more than one such pass take the MFMA kernels further down.
 //
 // lmh_rows: 512-thread workgroups; the pass's hidden rows (NB of them) are
 // staged in LDS as fp32; each wave streams whole vocab rows (lane l holds ids
@@ -37,6 +36,8 @@
 // lmh_chain (greedy chains, one thread per sequence) or lmh_tree (the EAGLE3
 // tree, one thread) applies the rule of llima_verify_greedy / llima_verify_tree
 // to the ids, again with no logits written.
+#include <type_traits>
+
 #include "common.hpp"
 #include "../../include/llima_sampler.h"
 
@@ -110,6 +111,17 @@ __device__ __forceinline__ void lmh_store_logit(const LmhParams& P, size_t i, fl
         ((uint16_t*)P.out_logits)[i] = v == v ? (uint16_t)(__float_as_uint(v) >> 16) : (uint16_t)0x7FC0u;
     else
         P.out_logits[i] = v;
+}
+
+// Logits i .. i + 3 (i a multiple of 4): one store.
+__device__ __forceinline__ void lmh_store_logits4(const LmhParams& P, size_t i, float4 x) {
+    if (P.logits_bf16) {
+        auto h = [](float v) { return v == v ? __float_as_uint(v) >> 16 : 0x7FC0u; };
+        const uint2 q = make_uint2(h(x.x) | h(x.y) << 16, h(x.z) | h(x.w) << 16);
+        *(uint2*)((uint16_t*)P.out_logits + i) = q;
+    } else {
+        *(float4*)(P.out_logits + i) = x;
+    }
 }
 
 #define LMH_LOG2E 1.44269504088896340736f
@@ -243,7 +255,7 @@ __global__ __launch_bounds__(LMH_WG) void lmh_rows(LmhParams P, int b0, int nb) 
 
 // ------------------------------------------------------------------ MFMA path
 // Batches wider than one GEMV pass: gfx950's v_mfma_f32_32x32x16_bf16 tiles,
-// the weight read once per pass of up to 256 hidden rows.  Lane l supplies row
+// the weight read once per pass of up to 128 (lmh_mfma) or 256 (lmh_tiles) rows.  Lane l supplies row
 // (A: a hidden row) or column (B: a vocab row) l % 32 and 8 consecutive values
 // of k; the k assignment only has to be the same for both operands, and step s
 // of a 64-id chunk gives lane half g the ids 16 s + 8 g .. 16 s + 8 g + 7, so
@@ -252,7 +264,7 @@ __global__ __launch_bounds__(LMH_WG) void lmh_rows(LmhParams P, int b0, int nb) 
 // is not the GEMV path's.
 typedef __bf16 lmh_b8 __attribute__((ext_vector_type(8)));
 typedef float lmh_acc __attribute__((ext_vector_type(16)));
-#define LMH_MB 256                     // hidden rows per pass at most
+#define LMH_MB 128                     // hidden rows of lmh_mfma's one pass at most
 
 __device__ __forceinline__ uint64_t lmh_key(float s, int n, int V) {
     return s == s && n < V ? ((uint64_t)f32_key(s) << 32) | (uint32_t)~(uint32_t)n : 0ull;
@@ -380,6 +392,8 @@ __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v
     }
 }
 
+#define LMH_KC 64                      // k per chunk; the H multiple the MFMA paths need
+
 // Workgroup tile: 32 NWN vocab rows x 64 WM hidden rows, 64 NWN WM threads.
 // Wave w computes vocab rows 32 (w % NWN) .. + 31 against hidden rows
 // 64 (w / NWN) .. + 63 (two 32 x 32 accumulators); the WM groups of waves share
@@ -389,8 +403,6 @@ __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v
 // one barrier per chunk).  The registers form a ring of R chunks, so R chunks
 // are in flight while one feeds the MFMAs: a chunk's loads are requested R
 // iterations before it is staged.
-#define LMH_KC 64                      // the H multiple the MFMA path needs
-
 template <int NWN, int WM, int R, int KC, bool SC>
 __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, int nb) {
     constexpr int NT = 64 * NWN * WM;                        // threads
@@ -503,6 +515,390 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
         lmh_logit_tile<1>(v, P);
         lmh_tile_out<1, SC>(P, v, ncol, wm * 64 + mt * 32, b0, nb, wv, r, g, tgv[mt]);
     }
+}
+
+// Requests 1 KB into LDS: lane l's 16 bytes at base + off go to dst + 16 l.
+__device__ __forceinline__ void lmh_dma(const uint8_t* base, uint32_t off, uint8_t* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + off),
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// An LDS write that does not wait for the requests in flight, as the
+// compiler's own writes to an array with requests do.
+__device__ __forceinline__ void lmh_lds_write(uint8_t* dst, uint2 v) {
+    const uint32_t a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dst;
+    asm volatile("ds_write_b64 %0, %1" ::"v"(a), "v"(v) : "memory");
+}
+
+// Waits until at most N of the wave's vector memory requests are in flight and
+// its LDS reads have returned, then for the workgroup.
+template <int N>
+__device__ __forceinline__ void lmh_wait_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+#define LMH_SLOT 64                    // vocab rows per key slot of lmh_tiles
+#define LMH_NV 256                     // vocab rows per tile of lmh_tiles
+#define LMH_CUS 256                    // workgroups of lmh_tiles: one per CU (its LDS)
+
+// f(0) .. f(N - 1) with compile-time arguments: for loops over accumulators
+// whose bodies are too long for the unroll pragma (a loop that stays puts the
+// accumulators in scratch memory).
+template <int I = 0, int N, class F>
+__device__ __forceinline__ void lmh_unrolled(std::integral_constant<int, N> n, F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        lmh_unrolled<I + 1>(n, f);
+    }
+}
+
+__device__ __forceinline__ float lmh_max3(float a, float b, float c) {
+    float d;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+
+// 32 sums of one lane as the argmax sees them (lmh_logit), in place; the two
+// decisions are taken once, the rounding is the hardware's (ties to even).
+__device__ __forceinline__ void lmh_logits32(const LmhParams& P, float (&x)[32]) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+    if (P.cap > 0.0f) {                                      // uniform
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            x[k] = P.cap * tanhf(x[k] / P.cap);
+            __builtin_amdgcn_sched_barrier(0);               // one at a time: interleaved, they spill
+        }
+    }
+    if (P.round_bf16) {                                      // uniform
+#pragma unroll
+        for (int k = 0; k < 32; k += 2) {
+            const f2 v = {x[k], x[k + 1]};
+            const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, h2));
+            x[k] = __uint_as_float(u << 16);
+            x[k + 1] = __uint_as_float(u & 0xFFFF0000u);
+        }
+    }
+}
+
+// The greatest of the two lanes' 64 logits (NaN only when all are) and the
+// first vocab row that has it, relative to the slot's; 255 when none has.
+// Lane half g holds, at k, row (k / 16) 32 + (k / 4 % 4) 8 + 4 g + k % 4.
+__device__ __forceinline__ int lmh_first_max(const float (&x)[32], int g, float& best) {
+    float m[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        m[q] = lmh_max3(x[q], x[q + 4], x[q + 8]);
+        m[q] = lmh_max3(m[q], x[q + 12], x[q + 16]);
+        m[q] = lmh_max3(m[q], x[q + 20], x[q + 24]);
+    }
+    const float a = lmh_max3(m[0], x[28], x[29]), b = lmh_max3(m[1], x[30], x[31]);
+    float c = lmh_max3(a, b, m[2]);
+    c = lmh_max3(c, m[3], m[3]);
+    best = lmh_max3(c, __shfl_xor(c, 32, 64), c);
+    int at = 255;
+#pragma unroll
+    for (int k = 31; k >= 0; --k) at = x[k] == best ? (k >> 4) * 32 + (k >> 2 & 3) * 8 + (k & 3) : at;
+    at = at == 255 ? 255 : at + 4 * g;
+    const int o = __shfl_xor(at, 32, 64);
+    return at < o ? at : o;
+}
+
+// lmh_tiles: batches of more rows than lmh_mfma (plain weight) or lmh_packed
+// hold in a pass.  A unit is 256 vocab rows against NM hidden rows; a workgroup
+// of four waves (one per SIMD, one workgroup per CU) runs through its units,
+// WVN waves along the vocab rows.  k goes in chunks of 64 ids; a chunk is
+// requested straight into LDS (1 KB per request, no registers), the weight RW
+// chunks deep and the hidden rows RX deep, and the requests run on into the
+// next unit, so that its first chunks arrive during the epilogue.  LDS rows are
+// 128 bytes with their 16-byte columns exchanged by row / 2 (the request's
+// source address does it), so fragment reads have no bank conflicts; a packed
+// weight's fragments lie in LDS as in memory.  Fragments are read one k-step
+// ahead of their MFMAs and the requests are spread over the k-steps: issued in
+// one burst they hold the wave's issue slot, and with it the matrix core, for
+// about half a chunk (B = 512 529 -> 490 us).  The MFMA takes the weight as its
+// row operand: a lane then has 32 of a hidden row's 64 logits of a key slot, so
+// that the epilogue works in registers with one exchange (lane ^ 32) instead of
+// a reduction over 32 lanes.  The sums' k order is lmh_mfma's: the logits are
+// the same bits.
+//
+// Bound: the matrix cores at B > 128 (B = 512, H = 4096, V = 128256: 538 GFLOP
+// in 432 us, 1.25 PFLOP/s; a library product of 8192^3 reaches 1.42), reading
+// the weight at B <= 128 (1.05 GB in 178 us, 5.9 TB/s).  Before: 696 us (plain)
+// and 1287 us (packed) at B = 512, 324 us (packed) at B = 128.
+template <int NM, int WVN, int RW, int RX, bool PK, bool SC>
+__global__ __launch_bounds__(256) void lmh_tiles(LmhParams P, const uint8_t* weight, int npass) {
+    constexpr int NV = LMH_NV, WMN = 4 / WVN;                // WMN: waves along the hidden rows
+    constexpr int VB = NV / WVN / 32, MB = NM / WMN / 32;    // 32 x 32 tiles per wave
+    constexpr int LW = NV / 32, LX = NM / 32;                // 1 KB requests per wave and chunk
+    constexpr int QI = (LX + LW + 3) / 4;                    // of them per k-step
+    constexpr int WB = NV * 128, XB = NM * 128;              // bytes of a staged chunk
+    // requests younger than the hidden ones of the chunk that is waited for
+    constexpr int FLY = LX * (RX - 2) + LW * (RX == RW ? RX - 2 : RX - 1);
+    static_assert(RX >= 2 && RX <= RW && VB % 2 == 0 && QI <= LX, "rings");
+    // one array: with two the compiler waits for every request before each LDS read
+    __shared__ __align__(1024) uint8_t sm[RW * WB + RX * XB];
+    uint8_t* const sw = sm;
+    uint8_t* const sx = sm + RW * WB;
+    const int t = (int)threadIdx.x, lane = t & 63, g = lane >> 5, r = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wn = wave % WVN, wm = wave / WVN;
+    const int H = P.H, V = P.V, NRB = (V + 31) / 32, nch = H / LMH_KC;
+    const int ntile = (V + NV - 1) / NV, nunit = ntile * npass, step_u = (int)gridDim.x;
+    // unit u: a vocab tile and a pass; the workgroups of one XCD (u % 8) take
+    // all passes of a tile one after the other
+    auto place = [&](int u, int& tile, int& pass) {
+        const int full = ntile & ~7;                         // tiles in whole groups of 8
+        if (u < full * npass) {
+            pass = (u >> 3) % npass;
+            tile = (u >> 3) / npass * 8 + (u & 7);
+        } else {
+            pass = (u - full * npass) / (ntile - full);
+            tile = full + (u - full * npass) % (ntile - full);
+        }
+    };
+    // The two request streams, weight and hidden: a unit, a chunk of it, the
+    // ring slot it goes to, and where the lane's requests read.
+    int uw = (int)blockIdx.x, cw = 0, lw = 0, ux = uw, cx = 0, lx = 0;
+    uint32_t ow[LW], ox[LX];
+    const uint8_t *bw, *bx;
+    auto set_w = [&]() {
+        int tile, pass;
+        place(uw, tile, pass);
+        const int n0 = tile * NV;
+        bw = PK ? weight + (size_t)(n0 / 32) * 8192 : weight + (size_t)n0 * H * 2;
+#pragma unroll
+        for (int q = 0; q < LW; ++q) {
+            if constexpr (PK) {                              // fragment (f / 4, f % 4) of the chunk
+                const int f = wave + 4 * q, rb = n0 / 32 + f / 4;
+                ow[q] = (uint32_t)((rb < NRB ? rb : NRB - 1) - n0 / 32) * 8192u +
+                        (uint32_t)(f & 3) * 1024u + (uint32_t)lane * 16u;
+            } else {
+                const int row = 8 * (wave + 4 * q) + (lane >> 3);
+                ow[q] = (uint32_t)(n0 + row < V ? row : V - 1 - n0) * (uint32_t)H * 2u +
+                        (uint32_t)(((lane & 7) ^ (row >> 1 & 7)) * 16);
+            }
+        }
+    };
+    auto set_x = [&]() {
+        int tile, pass;
+        place(ux, tile, pass);
+        bx = (const uint8_t*)P.hidden + (size_t)pass * NM * H * 2;
+        const int nb = P.B - pass * NM;
+#pragma unroll
+        for (int q = 0; q < LX; ++q) {
+            const int row = 8 * (wave + 4 * q) + (lane >> 3);
+            ox[q] = (uint32_t)(row < nb ? row : 0) * (uint32_t)H * 2u +
+                    (uint32_t)(((lane & 7) ^ (row >> 1 & 7)) * 16);
+        }
+    };
+    // past its last unit a stream repeats its last chunk (nobody reads it)
+    auto next_w = [&]() {
+        lw = lw + 1 == RW ? 0 : lw + 1;
+        if (++cw == nch) {
+            if (uw + step_u < nunit) { uw += step_u; cw = 0; set_w(); }
+            else cw = nch - 1;
+        }
+    };
+    auto next_x = [&]() {
+        lx = lx + 1 == RX ? 0 : lx + 1;
+        if (++cx == nch) {
+            if (ux + step_u < nunit) { ux += step_u; cx = 0; set_x(); }
+            else cx = nch - 1;
+        }
+    };
+    // requests k0 .. k1 - 1 of the streams' chunks, the hidden ones first
+    auto issue = [&](int k0, int k1) {
+        const uint8_t* gx = bx + (size_t)cx * 128;
+        const uint8_t* gw = PK ? bw + (size_t)(cw >> 1) * NRB * 8192 + (cw & 1) * 4096 : bw + (size_t)cw * 128;
+#pragma unroll
+        for (int k = k0; k < k1; ++k) {
+            if (k < LX) lmh_dma(gx, ox[k], sx + lx * XB + (wave + 4 * k) * 1024);
+            else if (k < LX + LW) lmh_dma(gw, ow[k - LX], sw + lw * WB + (wave + 4 * (k - LX)) * 1024);
+        }
+    };
+    const uint32_t rl = (uint32_t)(r * 128 + ((g ^ (r >> 1 & 7)) << 4));
+    auto read_frags = [&](const uint8_t* wb, const uint8_t* xb, int s, lmh_b8 (&fa)[MB], lmh_b8 (&fb)[VB]) {
+#pragma unroll
+        for (int j = 0; j < VB; ++j)
+            fb[j] = PK ? *(const lmh_b8*)(wb + ((wn * VB + j) * 4 + s) * 1024 + lane * 16)
+                       : *(const lmh_b8*)(wb + (wn * VB + j) * 4096 + (rl ^ (uint32_t)(s * 32)));
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+            fa[i] = *(const lmh_b8*)(xb + (wm * MB + i) * 4096 + (rl ^ (uint32_t)(s * 32)));
+    };
+    auto mfmas = [&](lmh_acc (&acc)[MB][VB], const lmh_b8 (&fa)[MB], const lmh_b8 (&fb)[VB]) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < VB; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    };
+    // A k-step: its MFMAs, between them the next k-step's LDS reads and QI requests.
+    auto step = [&](lmh_acc (&acc)[MB][VB], const uint8_t* wb, const uint8_t* xb, int s, lmh_b8 (&na)[MB], lmh_b8 (&nf)[VB],
+                    const lmh_b8 (&fa)[MB], const lmh_b8 (&fb)[VB], int k0) {
+        read_frags(wb, xb, s, na, nf);
+        issue(k0, k0 + QI);
+        mfmas(acc, fa, fb);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // MFMA
+#pragma unroll
+        for (int q = 0; q < MB + VB; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < QI; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);   // request
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    set_w();
+    set_x();
+#pragma unroll
+    for (int e = 1; e < RW; ++e) {                           // chunks 0 .. RW - 2 and 0 .. RX - 2
+        const bool x = e > RW - RX;
+        issue(x ? 0 : LX, LX + LW);
+        if (x) next_x();
+        next_w();
+    }
+    int ws = 0, xs = 0;                                      // ring slots of the chunk being read
+    lmh_b8 fa0[MB], fb0[VB], fa1[MB], fb1[VB];
+    lmh_wait_barrier<FLY>();                                 // chunk 0 has landed
+    issue(0, QI);
+    read_frags(sw, sx, 0, fa0, fb0);
+    for (int u = (int)blockIdx.x; u < nunit; u += step_u) {
+        lmh_acc acc[MB][VB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < VB; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+        uint8_t* spare = sw;
+        int c = 0;
+        do {
+            const uint8_t* wb = sw + ws * WB;
+            const uint8_t* xb = sx + xs * XB;
+            __builtin_amdgcn_sched_barrier(0);
+            step(acc, wb, xb, 1, fa1, fb1, fa0, fb0, QI);
+            step(acc, wb, xb, 2, fa0, fb0, fa1, fb1, 2 * QI);
+            step(acc, wb, xb, 3, fa1, fb1, fa0, fb0, 3 * QI);
+            spare = sw + ws * WB;
+            ws = ws + 1 == RW ? 0 : ws + 1;
+            xs = xs + 1 == RX ? 0 : xs + 1;
+            next_x();
+            next_w();
+            // the next chunk (of this unit or the next one) has landed, and
+            // this one's slots, which the streams take next, are read
+            lmh_wait_barrier<FLY>();
+            __builtin_amdgcn_sched_barrier(0);
+            step(acc, sw + ws * WB, sx + xs * XB, 0, fa0, fb0, fa1, fb1, 0);
+        } while (++c < nch);                                 // one exit: with two the accumulators are copied
+        // Epilogue: lane (r, g) has, for hidden row r of block i, half of the
+        // vocab rows of each of the wave's slots (the other half is the lane's
+        // with the other g).  bf16 logits leave through the last chunk's slot
+        // of the weight ring, 4 KB per wave, as whole 128-byte pieces of rows
+        // (its next requests come after a step's QI, which are hidden ones).
+        int el = lane;                                       // as if new here: the epilogue's addresses are
+        asm volatile("" : "+v"(el));                         // not computed before the loop, and do not spill
+        const int g = el >> 5, r = el & 31, lane = el;
+        int tile, pass;
+        place(u, tile, pass);
+        const int n0 = tile * NV, b0 = pass * NM, nb = P.B - b0 < NM ? P.B - b0 : NM;
+        uint8_t* const tr = spare + wave * 4096;
+        const bool put16 = P.out_logits && P.logits_bf16;    // uniform
+        // The sums stay in the accumulator registers until their slot reads
+        // them (left to the compiler all are moved at once, which spills);
+        // an MFMA's result may be read 19 wait states after it.
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        lmh_unrolled(std::integral_constant<int, MB>{}, [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            const int m0 = (wm * MB + i) * 32, m = m0 + r;
+            const bool row = m < nb;
+            const int32_t tg = SC && row ? P.targets[b0 + m] : -1;
+            lmh_unrolled(std::integral_constant<int, VB / 2>{}, [&](auto jc) __attribute__((always_inline)) {
+                constexpr int jp = decltype(jc)::value;
+                __builtin_amdgcn_sched_barrier(0);           // one slot's values at a time
+                const int lc = (wn * VB + 2 * jp) * 32;      // the slot's first column of the tile
+                const int n = n0 + lc, left = V - n;
+                float x[32];
+#pragma unroll
+                for (int k = 0; k < 32; ++k)
+                    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x[k]) : "a"(acc[i][2 * jp + (k >> 4)][k & 15]));
+                auto col = [&](int k) { return (k >> 4) * 32 + (k >> 2 & 3) * 8 + 4 * g + (k & 3); };
+                lmh_logits32(P, x);
+                if (put16) {
+                    auto h = [](float v) { return v == v ? __float_as_uint(v) >> 16 : 0x7FC0u; };
+#pragma unroll
+                    for (int k = 0; k < 32; k += 4)
+                        lmh_lds_write(tr + r * 128 + (((k >> 2) ^ (r >> 1 & 7)) << 4) + 8 * g,
+                                      make_uint2(h(x[k]) | h(x[k + 1]) << 16, h(x[k + 2]) | h(x[k + 3]) << 16));
+                    uint16_t* out = (uint16_t*)P.out_logits + n;
+                    if (V % 8 == 0) {                        // 16-byte pieces, wholly inside or outside
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const int mr = 8 * q + (lane >> 3), ch = lane & 7;
+                            const llima_u32x4 w = *(const llima_u32x4*)(tr + mr * 128 + ((ch ^ (mr >> 1 & 7)) << 4));
+                            if (m0 + mr < nb && ch * 8 < left)
+                                *(llima_u32x4*)(out + (size_t)(b0 + m0 + mr) * V + ch * 8) = w;
+                        }
+                    } else {
+                        for (int mr = 0; mr < 32 && m0 + mr < nb; ++mr) {
+                            const uint16_t w = *(const uint16_t*)(tr + mr * 128 + (((lane >> 3) ^ (mr >> 1 & 7)) << 4) + (lane & 7) * 2);
+                            if (lane < left) out[(size_t)(b0 + m0 + mr) * V + lane] = w;
+                        }
+                    }
+                } else if (P.out_logits) {                   // fp32 logits, 4 columns at a time
+#pragma unroll
+                    for (int k = 0; k < 32; k += 4) {
+                        float* o = P.out_logits + (size_t)(b0 + m) * V + n + col(k);
+                        if (row && V % 4 == 0) {
+                            if (col(k) < left) *(float4*)o = make_float4(x[k], x[k + 1], x[k + 2], x[k + 3]);
+                        } else if (row) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (col(k + e) < left) o[e] = x[k + e];
+                        }
+                    }
+                }
+                if (left < LMH_SLOT) {                       // uniform: columns past the vocabulary
+#pragma unroll
+                    for (int k = 0; k < 32; ++k) x[k] = col(k) < left ? x[k] : __builtin_nanf("");
+                }
+                float best;
+                const int at = lmh_first_max(x, g, best);
+                const size_t slot = (size_t)(b0 + m) * P.NW + n / LMH_SLOT;
+                if (row && g == 0)
+                    P.keys[slot] = at < 255 ? ((uint64_t)f32_key(best) << 32) | (uint32_t)~(uint32_t)(n + at) : 0ull;
+                if constexpr (SC) {
+                    if (left < LMH_SLOT) {                   // uniform
+#pragma unroll
+                        for (int k = 0; k < 32; ++k) x[k] = col(k) < left ? x[k] : -__builtin_inff();
+                    }
+                    const float mw = best > -__builtin_inff() ? best : 0.0f;
+                    float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int k = 0; k < 32; ++k) e[k & 3] += __builtin_amdgcn_exp2f((x[k] - mw) * LMH_LOG2E);
+                    float s = (e[0] + e[1]) + (e[2] + e[3]);
+                    s += __shfl_xor(s, 32, 64);
+                    if (row && g == 0) P.sums[slot] = s;
+                    const int ts = tg - n;                   // the target's column of the slot
+                    const bool hit = tg >= 0 && ts >= 0 && ts < LMH_SLOT && ts < left && (ts >> 2 & 1) == g;
+                    if (__any(hit)) {
+                        float v = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 32; ++k) v = ts == col(k) ? x[k] : v;
+                        if (hit) P.tval[b0 + m] = v;
+                    }
+                }
+            });
+        });
+        if (put16) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the slot is free again
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // no request outlives the workgroup
 }
 
 // One workgroup per hidden row: the greatest key over the waves (16 loads per
@@ -822,11 +1218,15 @@ static int lmh_rows_per_pass(int H) {
 
 using namespace llima;
 
-// Key slots per hidden row of the MFMA kernel: one per 32 vocab rows, in
-// whole 256-row tiles (a grid of 128-row tiles writes 0 to the up to 4 slots
-// it leaves).
+// Key slots per hidden row of lmh_mfma, one per 32 vocab rows, in whole
+// 256-row tiles (a grid of 128-row tiles writes 0 to the up to 4 slots it
+// leaves), and of lmh_tiles, one per 64.
 static int lmh_mfma_waves(int V) {
     return (V + 255) / 256 * 8;
+}
+
+static int lmh_tile_slots(int V) {
+    return (V + LMH_NV - 1) / LMH_NV * (LMH_NV / LMH_SLOT);
 }
 
 static int lmh_plain_slots(int V) {
@@ -870,21 +1270,42 @@ static int lmh_check_plain(const void* hidden, const void* weight, int32_t B, in
     return LLIMA_OK;
 }
 
+// A batch through lmh_tiles, over a plain or a packed weight: one pass of 128
+// rows, or passes of 256 that share the weight through the L2 of an XCD.
+template <bool PK, bool SC>
+static void lmh_run_tiles(LmhParams& P, const uint8_t* w, hipStream_t st) {
+    const int ntile = (P.V + LMH_NV - 1) / LMH_NV;
+    P.NW = lmh_tile_slots(P.V);
+    const int npass = P.B <= 128 ? 1 : (P.B + 255) / 256;
+    const int64_t nunit = (int64_t)ntile * npass;
+    const dim3 g((uint32_t)(nunit < LMH_CUS ? nunit : LMH_CUS));
+    if constexpr (PK) {
+        if (P.B <= 128) {
+            hipLaunchKernelGGL((lmh_tiles<128, 4, 3, 3, PK, SC>), g, dim3(256), 0, st, P, w, npass);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((lmh_tiles<256, 2, 3, 2, PK, SC>), g, dim3(256), 0, st, P, w, npass);
+}
+
 // The passes over the plain weight (MFMA tiles, or the matrix-vector rows
 // kernel) and the finish: lmh_finish, or lmh_score_finish with SC.
 template <bool SC>
 static int lmh_run_plain(LmhParams& P, hipStream_t st) {
     const int B = P.B, H = P.H, V = P.V;
-    if ((B > lmh_rows_per_pass(H) || H > LMH_MAX_H) && H % LMH_KC == 0) {   // MFMA tiles
-        P.NW = lmh_mfma_waves(V);
-        const dim3 g128((uint32_t)((V + 127) / 128));
-        for (int b0 = 0; b0 < B; b0 += LMH_MB) {
-            const int nb = B - b0 < LMH_MB ? B - b0 : LMH_MB;
-            // 128 vocab rows per workgroup; the narrowest tile that holds the
-            // pass: 64, 128 or 256 hidden rows
-            if (nb <= 64) hipLaunchKernelGGL((lmh_mfma<4, 1, 4, LMH_KC, SC>), g128, dim3(256), 0, st, P, b0, nb);
-            else if (nb <= 128) hipLaunchKernelGGL((lmh_mfma<4, 2, 2, LMH_KC, SC>), g128, dim3(512), 0, st, P, b0, nb);
-            else hipLaunchKernelGGL((lmh_mfma<4, 4, 2, LMH_KC, SC>), g128, dim3(1024), 0, st, P, b0, nb);
+    if ((B > lmh_rows_per_pass(H) || H > LMH_MAX_H) && H % LMH_KC == 0) {   // MFMA paths
+        // Up to 128 rows one pass of lmh_mfma: there both kernels are bound by
+        // reading 128-byte pieces of the plain weight's rows, and lmh_mfma has
+        // more of them in flight (B = 64 212 against 238 us, B = 128 235
+        // against 256, H = 4096, V = 128256).  Above, lmh_tiles (B = 256 294
+        // against 350 us, B = 512 436 against 696).
+        if (B > LMH_MB) {
+            lmh_run_tiles<false, SC>(P, (const uint8_t*)P.weight, st);
+        } else {
+            P.NW = lmh_mfma_waves(V);
+            const dim3 g128((uint32_t)((V + 127) / 128));
+            if (B <= 64) hipLaunchKernelGGL((lmh_mfma<4, 1, 4, LMH_KC, SC>), g128, dim3(256), 0, st, P, 0, B);
+            else hipLaunchKernelGGL((lmh_mfma<4, 2, 2, LMH_KC, SC>), g128, dim3(512), 0, st, P, 0, B);
         }
     } else {
         P.NW = lmh_waves(V);
@@ -1102,7 +1523,8 @@ extern "C" size_t llima_lm_head_packed_bytes(int32_t V, int32_t H) {
 
 static int lmp_slots(int V) {
     const int g1 = lmp_groups(V, LMP_WR1), g2 = lmp_groups(V, LMP_WR2);
-    return (g1 > g2 ? g1 : g2) * LMP_WAVES;
+    const int n = (g1 > g2 ? g1 : g2) * LMP_WAVES;
+    return n > lmh_tile_slots(V) ? n : lmh_tile_slots(V);
 }
 
 extern "C" size_t llima_lm_head_argmax_packed_workspace_bytes(int32_t B, int32_t H, int32_t V) {
@@ -1134,15 +1556,18 @@ static int lmh_run_packed(LmhParams& P, const uint8_t* packed, hipStream_t st) {
     const int B = P.B, V = P.V;
     const int ng1 = lmp_groups(V, LMP_WR1), ng2 = lmp_groups(V, LMP_WR2);
     P.NW = lmp_slots(V);
-    for (int b0 = 0; b0 < B; b0 += LMP_MB) {
-        const int nb = B - b0 < LMP_MB ? B - b0 : LMP_MB;
-        if (nb <= 32)
-            hipLaunchKernelGGL((lmh_packed<1, LMP_WR1, LMP_R1, LMP_KR, SC>), dim3(ng1), dim3(LMP_WG), 0,
-                               st, P, packed, b0, nb);
-        else
-            hipLaunchKernelGGL((lmh_packed<2, LMP_WR2, LMP_R2, LMP_KR, SC>), dim3(ng2), dim3(LMP_WG), 0,
-                               st, P, packed, b0, nb);
-    }
+    // Up to 64 rows a wave streams its own vocab rows into registers (165 us at
+    // B = 64, H = 4096, V = 128256); above, where that kernel would read the
+    // weight again per 64 rows (B = 128 324 us, B = 256 646, B = 512 1287),
+    // lmh_tiles (178, 245 and 432 us).
+    if (B > LMP_MB)
+        lmh_run_tiles<true, SC>(P, packed, st);
+    else if (B <= 32)
+        hipLaunchKernelGGL((lmh_packed<1, LMP_WR1, LMP_R1, LMP_KR, SC>), dim3(ng1), dim3(LMP_WG), 0,
+                           st, P, packed, 0, B);
+    else
+        hipLaunchKernelGGL((lmh_packed<2, LMP_WR2, LMP_R2, LMP_KR, SC>), dim3(ng2), dim3(LMP_WG), 0,
+                           st, P, packed, 0, B);
     if (SC) hipLaunchKernelGGL(lmh_score_finish, dim3((uint32_t)B), dim3(LLIMA_WG), 0, st, P);
     else hipLaunchKernelGGL(lmh_finish, dim3((uint32_t)B), dim3(LLIMA_WG), 0, st, P);
     return hipGetLastError() == hipSuccess ? LLIMA_OK : LLIMA_E_HIP;

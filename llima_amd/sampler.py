@@ -539,7 +539,8 @@ class PackedLmHead:
     vocab rows x 16 ids, zero rows up to a multiple of 32, 8 KB groups per 32
     rows and 128 ids), so that each wave streams contiguous memory straight
     into the matrix cores.  `data` is the uint8 device tensor; V and H are the
-    weight's shape.  It is read once per 64 hidden rows."""
+    weight's shape.  It is read once per pass: up to 64 hidden rows, up to 128,
+    or 256 of a wider batch."""
 
     def __init__(self, data: torch.Tensor, V: int, H: int):
         self.data, self.V, self.H = data, V, H
