@@ -39,6 +39,11 @@ namespace llima {
 #define TK_PAD(e) ((e) + ((e) >> 4))      // LDS slot of tile element e (conflict-free rows)
 #define TK_CAP 4096                       // candidates of a tile held for the replay
 #define TK_MAXK 32                        // the reference's limit on k
+#define TK_PART_K 16                      // k at most for rows split into parts
+#define TK_PART 4096                      // values of a part
+#define TK_PARTS 64                       // parts of a row at most
+#define TK_PSLOTS 256                     // a part's slots: the count, then its candidates
+#define TK_PSTAGE 8                       // parts whose first candidates are staged together
 #define TREE_WG 256
 #define TREE_MAX_NODES 16384              // node scores the finish stages in LDS
 
@@ -47,7 +52,7 @@ namespace llima {
 // level's scores, the parent groups, every node's score and token, the draft
 // attention mask, and the per-row top-k of the level being grown.
 struct TreeLayout {
-    size_t score, parent, node_score, node_tok, mask, row_idx, row_val, total;
+    size_t score, parent, node_score, node_tok, mask, row_idx, row_val, cand, total;
 };
 
 __host__ __device__ inline size_t tree_take(size_t* o, size_t bytes) {
@@ -67,6 +72,7 @@ __host__ __device__ inline TreeLayout tree_layout(int K, int depth) {
     L.mask = tree_take(&o, 4 * (size_t)K * K * depth);
     L.row_idx = tree_take(&o, 4 * (size_t)K * K);
     L.row_val = tree_take(&o, 4 * (size_t)K * K);
+    L.cand = tree_take(&o, K <= TK_PART_K ? 8 * (size_t)K * TK_PARTS * TK_PSLOTS : 0);
     L.total = o;
     return L;
 }
@@ -89,6 +95,8 @@ struct TreeParams {
     int32_t* out_pos;        // [N]
     int32_t* out_retrieve;   // [N][N]
     int32_t* out_dims;       // [2]
+    int32_t parts;           // parts per row (0: rows not split)
+    int32_t bf16;            // split rows: bf16 values
 };
 
 template <typename T>
@@ -334,7 +342,7 @@ __device__ __forceinline__ void topk_row_generic(const TL* rowp, int cols, int k
 // onto +0; no NaN is ever in the heap on this path).  Each thread's k-th
 // largest key comes from a sorted list of its TK_FAST_K largest (one max/min
 // pair per list entry and value).
-#define TK_FAST_K 8
+#define TK_FAST_K 16                      // keys a register heap holds at most
 #define TK_VPT 16
 #define TK_FTILE (TK_WG * TK_VPT)
 
@@ -770,18 +778,250 @@ __device__ __forceinline__ bool heap_small_k(const float* x, int n, int k, int32
     }
 }
 
-// Level 0: the root row's top K, their log-softmax as the scores, their
-// mapped tokens; parent group 0; the draft mask starts as the K x K identity.
-template <typename TL>
-__global__ __launch_bounds__(TK_WG) void eagle3_begin_kernel(TreeParams P) {
-    __shared__ TopkShared sh;
-    __shared__ float lp[TK_MAXK], ex[TK_MAXK], shift[1];
+// The N largest keys of two descending lists (N a power of two) into a: the
+// pairwise maxima of a and the reversed b are those N keys as a bitonic
+// sequence, which log2 N exchanges sort.
+template <int N>
+__device__ __forceinline__ void tk_list_merge(uint32_t (&a)[N], const uint32_t (&b)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) a[i] = a[i] > b[N - 1 - i] ? a[i] : b[N - 1 - i];
+#pragma unroll
+    for (int s = N / 2; s > 0; s >>= 1)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if ((i & s) == 0) {
+                const uint32_t hi = a[i] > a[i + s] ? a[i] : a[i + s], lo = a[i] > a[i + s] ? a[i + s] : a[i];
+                a[i] = hi;
+                a[i + s] = lo;
+            }
+}
+
+// ------------------------------------------------------------------ rows split into parts
+// A tree level's rows (k <= TK_PART_K, at most TK_PARTS parts): one 256-thread
+// workgroup per 4096 values finds the values that can enter the row's heap,
+// those that exceed the k-th largest value of the part before them (~40 of
+// 4096), and writes them in id order to the part's slots; the level's last
+// kernel replays each row's parts in order, a wavefront per row.  One
+// workgroup per row instead runs ~900 vector instructions per thread on one
+// CU.  A part with more of them than slots (ascending values) says so in its
+// count, and its values are replayed one by one, as are all values of a row
+// with a NaN among its first k.
+template <typename TL, int KC>
+__global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
+    constexpr int NQ = TK_VPT * (int)sizeof(TL) / 16;
+    constexpr int N = KC <= 1 ? 1 : KC <= 2 ? 2 : KC <= 4 ? 4 : KC <= 8 ? 8 : 16;
+    __shared__ uint32_t wlist[TREE_WG / 64][N], wcnt[TREE_WG / 64];
     const TreeLayout L = tree_layout(P.K, P.depth);
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int row = (int)blockIdx.y, part = (int)blockIdx.x;
+    const TL* rowp = (const TL*)P.x + (size_t)row * P.row_stride;
+    const int ib = part * TK_PART + t * TK_VPT;
+    llima_u32x4 q[NQ];
+    tk_raw<TL>(rowp, ib, P.cols, P.vec != 0, q);
+    uint32_t kk[TK_VPT], Lk[TK_FAST_K];
+    tk_keys<TL>(q, kk);
+#pragma unroll
+    for (int i = 0; i < TK_FAST_K; ++i) Lk[i] = 0u;
+#pragma unroll
+    for (int e = 0; e < TK_VPT; ++e) tk_list_put<KC>(Lk, kk[e]);
+    // the KC largest keys of all earlier threads: a scan over the lanes, then
+    // the earlier waves' lists
+    uint32_t A[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) A[i] = Lk[i];
+    auto scan_step = [&](auto dpp) {
+        uint32_t B[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) B[i] = dpp(A[i]);
+        tk_list_merge<N>(A, B);
+    };
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_SHR(1), 0xF, true>(0u, v); });
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_SHR(2), 0xF, true>(0u, v); });
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_SHR(4), 0xF, true>(0u, v); });
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_SHR(8), 0xF, true>(0u, v); });
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_BCAST15, 0xA, false>(0u, v); });
+    scan_step([](uint32_t v) { return dpp32<DPP_ROW_BCAST31, 0xC, false>(0u, v); });
+    if (lane == 63) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) wlist[wave][i] = A[i];
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const uint32_t v = (uint32_t)__shfl_up((int)A[i], 1);
+        A[i] = lane == 0 ? 0u : v;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) {
+        uint32_t B[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) B[i] = wlist[w][i];
+        tk_list_merge<N>(A, B);
+    }
+    // a value enters when it exceeds the k-th largest before it (ids below k
+    // start the heap and are not written)
+#pragma unroll
+    for (int i = 0; i < TK_FAST_K; ++i) Lk[i] = i < N ? A[i < N ? i : 0] : 0u;
+    uint32_t cmask = 0;
+#pragma unroll
+    for (int e = 0; e < TK_VPT; ++e) {
+        cmask |= ib + e >= KC && kk[e] > Lk[KC - 1] ? 1u << e : 0u;
+        tk_list_put<KC>(Lk, kk[e]);
+    }
+    const uint32_t cnt = (uint32_t)__popc(cmask);
+    const uint32_t ci = wave_incl_scan_u32(cnt);
+    if (lane == 63) wcnt[wave] = ci;
+    __syncthreads();
+    uint32_t off = ci - cnt, total = 0;
+    for (int w = 0; w < TREE_WG / 64; ++w) {
+        off += w < wave ? wcnt[w] : 0u;
+        total += wcnt[w];
+    }
+    uint64_t* slots = st<uint64_t>(P, L.cand) + ((size_t)row * TK_PARTS + part) * TK_PSLOTS;
+#pragma unroll
+    for (int e = 0; e < TK_VPT; ++e)
+        if ((cmask >> e) & 1u) {
+            if (off < TK_PSLOTS - 1) slots[1 + off] = ((uint64_t)kk[e] << 32) | (uint32_t)(ib + e);
+            ++off;
+        }
+    if (t == 0) slots[0] = total;
+}
+
+// The heap of one row from its parts' candidates, by one wavefront (every lane
+// alike), then the reference's selection sort: out_i / out_v [KC] (LDS).
+template <int KC>
+__device__ __forceinline__ void parts_replay(const TreeParams& P, const TreeLayout& L, int row,
+                                             uint64_t (&stage)[TK_PSTAGE][64], int32_t* out_i,
+                                             float* out_v) {
+    const int lane = (int)lane_id();
+    const int64_t r0 = (int64_t)row * P.row_stride;
+    auto load = [&](int i) {                                // the row's value i
+        return P.bf16 ? tk_load<uint16_t>((const uint16_t*)P.x + r0, i) : tk_load<float>((const float*)P.x + r0, i);
+    };
+    const uint64_t* slots = st<uint64_t>(P, L.cand) + (size_t)row * TK_PARTS * TK_PSLOTS;
+    // the first 64 candidates of TK_PSTAGE parts, requested together
+    auto fetch = [&](int p0) {
+        uint64_t c[TK_PSTAGE];
+#pragma unroll
+        for (int i = 0; i < TK_PSTAGE; ++i) {
+            const int p = p0 + i < P.parts ? p0 + i : P.parts - 1;
+            c[i] = slots[(size_t)p * TK_PSLOTS + 1 + lane];
+        }
+#pragma unroll
+        for (int i = 0; i < TK_PSTAGE; ++i) stage[i][lane] = c[i];
+    };
+    const uint32_t pn = lane < P.parts ? (uint32_t)slots[(size_t)lane * TK_PSLOTS] : 0u;
+    const float f0 = lane < KC ? load(lane) : 0.0f;
+    const bool nan0 = ballot(f0 != f0) != 0ull;             // uniform
+    if (nan0) {                                             // NaNs in the heap: float compares
+        float hv = f0;
+        int32_t hi = lane;
+        for (int j = KC / 2 - 1; j >= 0; --j) heap_sift(hv, hi, j, KC);
+        float root = rdl_f(hv, 0);
+        for (int g = KC; g < P.cols; g += 64) {
+            const float x = g + lane < P.cols ? load(g + lane) : __builtin_nanf("");
+            uint64_t m = ballot(x > root);
+            while (m) {
+                const int Ln = __builtin_ctzll(m);
+                hv = wrl_f(hv, rdl_f(x, Ln), 0);
+                hi = wrl_i(hi, g + Ln, 0);
+                heap_sift(hv, hi, 0, KC);
+                root = rdl_f(hv, 0);
+                m = ballot(x > root) & (Ln == 63 ? 0ull : (~0ull << (Ln + 1)));
+            }
+        }
+        for (int a = 0; a < KC; ++a) {
+            int m = a;
+            float vm = rdl_f(hv, a);
+            for (int b = a + 1; b < KC; ++b) {
+                const float vb = rdl_f(hv, b);
+                if (vb > vm) { m = b; vm = vb; }
+            }
+            const int32_t im = rdl_i(hi, m);
+            if (lane == 0) { out_v[a] = vm; out_i[a] = im; }
+            hv = wrl_f(hv, rdl_f(hv, a), m);
+            hi = wrl_i(hi, rdl_i(hi, a), m);
+        }
+        return;
+    }
+    uint32_t hk[TK_FAST_K];
+    int32_t hi[TK_FAST_K];
+#pragma unroll
+    for (int i = 0; i < TK_FAST_K; ++i) {
+        hk[i] = i < KC ? (uint32_t)__builtin_amdgcn_readlane((int)f32_key(f0), i) : 0u;
+        hi[i] = i;
+    }
+    uheap_build<KC, KC / 2 - 1>(hk, hi);
+    uint32_t root = hk[0];
+    // One copy of the replay: the code runs once per row, so its length is
+    // instruction fetch (unrolled over the parts it took 113 us).
+#pragma unroll 1
+    for (int p = 0; p < P.parts; ++p) {
+        if (p % TK_PSTAGE == 0) fetch(p);
+        const uint32_t stored = (uint32_t)__builtin_amdgcn_readlane((int)pn, p);
+        const bool raw = stored > TK_PSLOTS - 1;            // not all stored: the part's values
+        const int base = p * TK_PART;
+        const int n = !raw ? (int)stored : P.cols - base < TK_PART ? P.cols - base : TK_PART;
+#pragma unroll 1
+        for (int g = 0; g < n; g += 64) {                   // 64 values in id order (key 0: none)
+            const int e = g + lane;
+            uint32_t x = 0u;
+            int32_t xj = base + e;
+            if (raw) {
+                const float f = e < n ? load(base + e) : __builtin_nanf("");
+                x = xj >= KC && f == f ? f32_key(f) : 0u;
+            } else {
+                const uint64_t v = g == 0 ? stage[p % TK_PSTAGE][lane]
+                                          : slots[(size_t)p * TK_PSLOTS + 1 + (e < n ? e : g)];
+                x = e < n ? (uint32_t)(v >> 32) : 0u;
+                xj = (int32_t)(uint32_t)v;
+            }
+            uint64_t m = ballot(x > root);
+            while (m) {
+                const int Ln = __builtin_ctzll(m);
+                hk[0] = (uint32_t)__builtin_amdgcn_readlane((int)x, Ln);
+                hi[0] = __builtin_amdgcn_readlane(xj, Ln);
+                uheap_sift<KC, 0>(hk, hi);
+                root = hk[0];
+                m = ballot(x > root) & (Ln == 63 ? 0ull : (~0ull << (Ln + 1)));
+            }
+        }
+    }
+    int32_t ri = 0;
+#pragma unroll
+    for (int a = 0; a < KC; ++a) {                          // the selection sort over the slots
+        uint32_t vm = hk[a];
+        int32_t im = hi[a];
+        int m = a;
+#pragma unroll
+        for (int b = a + 1; b < KC; ++b) {
+            const bool gt = hk[b] > vm;
+            vm = gt ? hk[b] : vm;
+            im = gt ? hi[b] : im;
+            m = gt ? b : m;
+        }
+        ri = lane == a ? im : ri;
+#pragma unroll
+        for (int b = a + 1; b < KC; ++b) {
+            hk[b] = m == b ? hk[a] : hk[b];
+            hi[b] = m == b ? hi[a] : hi[b];
+        }
+    }
+    if (lane < KC) {
+        out_i[lane] = ri;
+        out_v[lane] = load(ri);                // the row's own bits (-0 included)
+    }
+}
+
+// Level 0 from the root row's top K (res_i, res_v): their log-softmax as the
+// scores, their mapped tokens; parent group 0; the draft mask starts as the
+// K x K identity.
+__device__ __forceinline__ void begin_level(const TreeParams& P, const TreeLayout& L,
+                                            const int32_t* res_i, const float* res_v) {
+    __shared__ float lp[TK_MAXK], ex[TK_MAXK], shift[1];
     const int K = P.K, t = (int)threadIdx.x;
-    topk_row<TL>((const TL*)P.x, P.cols, K, P.vec != 0, sh);
-    logsoftmax_rows(sh.res_v, 1, K, ex, shift, lp);
+    logsoftmax_rows(res_v, 1, K, ex, shift, lp);
     if (t < K) {
-        const int32_t id = sh.res_i[t];
+        const int32_t id = res_i[t];
         const int32_t tok = id + P.d2t[id];
         st<float>(P, L.score)[t] = lp[t];
         st<float>(P, L.node_score)[t] = lp[t];
@@ -790,7 +1030,15 @@ __global__ __launch_bounds__(TK_WG) void eagle3_begin_kernel(TreeParams P) {
     }
     if (t == 0) st<int32_t>(P, L.parent)[0] = 0;
     const int mc = K * P.depth;
-    for (int e = t; e < K * mc; e += TK_WG) st<float>(P, L.mask)[e] = (e % mc) == e / mc ? 1.0f : 0.0f;
+    for (int e = t; e < K * mc; e += (int)blockDim.x)
+        st<float>(P, L.mask)[e] = (e % mc) == e / mc ? 1.0f : 0.0f;
+}
+
+template <typename TL>
+__global__ __launch_bounds__(TK_WG) void eagle3_begin_kernel(TreeParams P) {
+    __shared__ TopkShared sh;
+    topk_row<TL>((const TL*)P.x, P.cols, P.K, P.vec != 0, sh);
+    begin_level(P, tree_layout(P.K, P.depth), sh.res_i, sh.res_v);
 }
 
 // The top K of each of the K rows of a level, into the state.
@@ -806,37 +1054,41 @@ __global__ __launch_bounds__(TK_WG) void eagle3_rows_kernel(TreeParams P) {
     }
 }
 
-// Level `level` (1 .. depth-1) from the rows' top K: cumulative scores, the
-// best K of them, parent rows, next input ids, node lists, parent group, mask.
-__global__ __launch_bounds__(TREE_WG) void eagle3_combine_kernel(TreeParams P) {
-    __shared__ float cu[TK_MAXK * TK_MAXK];
-    __shared__ int32_t tok[TK_MAXK * TK_MAXK];
-    __shared__ float rv[TK_MAXK * TK_MAXK];
-    __shared__ float score[TK_MAXK], hv[TK_MAXK], bestv[TK_MAXK], shift[TK_MAXK];
-    __shared__ float ex[TK_MAXK * TK_MAXK];
-    __shared__ int32_t hi[TK_MAXK], best[TK_MAXK];
+// Level `level` (1 .. depth-1) from the rows' top K (row_i, row_v, in LDS or in
+// the state): cumulative scores, the best K of them, parent rows, next input
+// ids, node lists, parent group, mask.
+template <int KM>
+__device__ __forceinline__ void combine_level(const TreeParams& P, const TreeLayout& L,
+                                              const int32_t* row_i, const float* row_v) {
+    __shared__ float cu[KM * KM];
+    __shared__ int32_t tok[KM * KM];
+    __shared__ float rv[KM * KM];
+    __shared__ float score[KM], hv[KM], bestv[KM], shift[KM];
+    __shared__ float ex[KM * KM];
+    __shared__ int32_t hi[KM], best[KM];
     __shared__ uint32_t fast;
-    __shared__ float oldm[TK_MAXK * TK_MAXK * 16];
-    const TreeLayout L = tree_layout(P.K, P.depth);
-    const int K = P.K, KK = K * K, t = (int)threadIdx.x;
+    __shared__ float oldm[KM * KM * 16];
+    const int K = P.K, KK = K * K, t = (int)threadIdx.x, NT = (int)blockDim.x;
     const int i = P.level - 1;                    // the reference's loop counter
     const int mc = K * P.depth, acols = K * P.level;
-    for (int q = t; q < KK; q += TREE_WG) {
-        const int32_t id = st<int32_t>(P, L.row_idx)[q];
+    for (int q = t; q < KK; q += NT) {
+        const int32_t id = row_i[q];
         tok[q] = id + P.d2t[id];
-        rv[q] = st<float>(P, L.row_val)[q];
+        rv[q] = row_v[q];
     }
     if (t < K) score[t] = st<float>(P, L.score)[t];
-    for (int e = t; e < K * acols; e += TREE_WG)
+    for (int e = t; e < K * acols; e += NT)
         oldm[e] = st<float>(P, L.mask)[(e / acols) * mc + e % acols];
     __syncthreads();
     // each row's log-softmax plus the row's score (the reference's float steps)
     logsoftmax_rows(rv, K, K, ex, shift, cu);
-    for (int q = t; q < KK; q += TREE_WG) cu[q] = cu[q] + score[q / K];
+    for (int q = t; q < KK; q += NT) cu[q] = cu[q] + score[q / K];
     __syncthreads();
     // the best K of the K*K cumulative scores (the reference's heap)
     if (t < 64) {
-        const bool ok = heap_small_k(cu, KK, K, best, bestv);
+        bool ok;
+        if constexpr (KM <= TK_PART_K) ok = heap_small<KM>(cu, KK, best, bestv);   // KM == K
+        else ok = heap_small_k(cu, KK, K, best, bestv);
         if (t == 0) fast = ok ? 1u : 0u;
     }
     __syncthreads();
@@ -845,7 +1097,7 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_combine_kernel(TreeParams P) {
         __syncthreads();
     }
     const size_t nbase = (size_t)K + (size_t)i * KK;
-    for (int q = t; q < KK; q += TREE_WG) {
+    for (int q = t; q < KK; q += NT) {
         st<float>(P, L.node_score)[nbase + q] = cu[q];
         st<int32_t>(P, L.node_tok)[nbase + q] = tok[q];
     }
@@ -858,12 +1110,32 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_combine_kernel(TreeParams P) {
     }
     // the mask: row r = old row of its parent, then an identity block
     const int ncols = acols + K;
-    for (int e = t; e < K * ncols; e += TREE_WG) {
+    for (int e = t; e < K * ncols; e += NT) {
         const int r = e / ncols, c = e % ncols;
         const float v = c < acols ? oldm[(best[r] / K) * acols + c] : (c - acols == r ? 1.0f : 0.0f);
         st<float>(P, L.mask)[r * mc + c] = v;
         if (P.out_mask) P.out_mask[e] = v;
     }
+}
+
+__global__ __launch_bounds__(TREE_WG) void eagle3_combine_kernel(TreeParams P) {
+    const TreeLayout L = tree_layout(P.K, P.depth);
+    combine_level<TK_MAXK>(P, L, st<int32_t>(P, L.row_idx), st<float>(P, L.row_val));
+}
+
+// A level after eagle3_parts_kernel: wavefront r replays row r (K wavefronts,
+// at least four; the root row alone at level 0), then the level's combine.
+template <int KC>
+__global__ __launch_bounds__(64 * (KC < 4 ? 4 : KC)) void eagle3_level_kernel(TreeParams P) {
+    __shared__ int32_t row_i[KC * KC];
+    __shared__ float row_v[KC * KC];
+    __shared__ uint64_t stage[KC][TK_PSTAGE][64];
+    const TreeLayout L = tree_layout(P.K, P.depth);
+    const int w = (int)wave_id();
+    if (w < (P.level == 0 ? 1 : KC)) parts_replay<KC>(P, L, w, stage[w], row_i + w * KC, row_v + w * KC);
+    __syncthreads();
+    if (P.level == 0) begin_level(P, L, row_i, row_v);
+    else combine_level<KC>(P, L, row_i, row_v);
 }
 
 // The final tree: best `total` node scores, tokens, parents located among the
@@ -1018,6 +1290,45 @@ static bool tree_dims_ok(int32_t K, int32_t depth) {
     return nodes <= TREE_MAX_NODES && (int64_t)K * K * (depth > 1 ? depth - 1 : 1) <= 16384;
 }
 
+// Parts per row when a level's rows are split (0 when they are not: k past the
+// register heap, or more values than TK_PARTS parts hold).
+static int32_t tree_parts(int32_t K, int32_t Vd) {
+    const int32_t n = (Vd + TK_PART - 1) / TK_PART;
+    return K <= TK_PART_K && n <= TK_PARTS ? n : 0;
+}
+
+// A level's two kernels over split rows: the parts of `rows` rows, then the
+// replay with the rest of the level (level 0 or a later one).
+template <int KC>
+static void launch_parts_k(const TreeParams& P, int rows, hipStream_t st) {
+    const dim3 g(P.parts, rows);
+    if (P.bf16) hipLaunchKernelGGL((eagle3_parts_kernel<uint16_t, KC>), g, dim3(TREE_WG), 0, st, P);
+    else hipLaunchKernelGGL((eagle3_parts_kernel<float, KC>), g, dim3(TREE_WG), 0, st, P);
+    hipLaunchKernelGGL(eagle3_level_kernel<KC>, dim3(1), dim3(64 * (KC < 4 ? 4 : KC)), 0, st, P);
+}
+
+static void launch_parts(const TreeParams& P, int rows, hipStream_t st) {
+    switch (P.K) {
+        case 1: launch_parts_k<1>(P, rows, st); break;
+        case 2: launch_parts_k<2>(P, rows, st); break;
+        case 3: launch_parts_k<3>(P, rows, st); break;
+        case 4: launch_parts_k<4>(P, rows, st); break;
+        case 5: launch_parts_k<5>(P, rows, st); break;
+        case 6: launch_parts_k<6>(P, rows, st); break;
+        case 7: launch_parts_k<7>(P, rows, st); break;
+        case 8: launch_parts_k<8>(P, rows, st); break;
+        case 9: launch_parts_k<9>(P, rows, st); break;
+        case 10: launch_parts_k<10>(P, rows, st); break;
+        case 11: launch_parts_k<11>(P, rows, st); break;
+        case 12: launch_parts_k<12>(P, rows, st); break;
+        case 13: launch_parts_k<13>(P, rows, st); break;
+        case 14: launch_parts_k<14>(P, rows, st); break;
+        case 15: launch_parts_k<15>(P, rows, st); break;
+        case 16: launch_parts_k<16>(P, rows, st); break;
+        default: break;
+    }
+}
+
 extern "C" int llima_topk(const void* x, int32_t dtype, int32_t rows, int32_t cols,
                           int64_t row_stride, int32_t k, int32_t* out_idx, float* out_vals,
                           void* stream) {
@@ -1052,8 +1363,11 @@ extern "C" int llima_eagle3_tree_begin(const void* logits, int32_t dtype, int32_
     P.x = logits; P.cols = Vd; P.k = K; P.d2t = d2t; P.state = (char*)tree;
     P.K = K; P.depth = depth; P.out_inputs = out_input_ids;
     P.vec = rows_vec(logits, Vd, dtype);
+    P.parts = tree_parts(K, Vd);
+    P.bf16 = dtype == LLIMA_BF16;
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == LLIMA_F32)
+    if (P.parts) launch_parts(P, 1, st);
+    else if (dtype == LLIMA_F32)
         hipLaunchKernelGGL(eagle3_begin_kernel<float>, dim3(1), dim3(TK_WG), 0, st, P);
     else
         hipLaunchKernelGGL(eagle3_begin_kernel<uint16_t>, dim3(1), dim3(TK_WG), 0, st, P);
@@ -1075,7 +1389,13 @@ extern "C" int llima_eagle3_tree_grow(const void* logits, int32_t dtype, int32_t
     P.state = (char*)tree; P.K = K; P.depth = depth; P.level = level;
     P.out_inputs = out_input_ids; P.out_prow = out_parent_rows; P.out_mask = out_mask;
     P.vec = rows_vec(logits, row_stride, dtype);
+    P.parts = tree_parts(K, Vd);
+    P.bf16 = dtype == LLIMA_BF16;
     hipStream_t st = (hipStream_t)stream;
+    if (P.parts) {
+        launch_parts(P, K, st);
+        return hipGetLastError() == hipSuccess ? LLIMA_OK : LLIMA_E_HIP;
+    }
     if (dtype == LLIMA_F32)
         hipLaunchKernelGGL(eagle3_rows_kernel<float>, dim3(K), dim3(TK_WG), 0, st, P);
     else

@@ -131,3 +131,51 @@ def test_eagle3_tree_ties_and_shapes(gpu, oracle):
         d2t = rng.integers(0, 1000, Vd).astype(np.int32)
         _run_tree(gpu, oracle, wl.f32_to_bf16_bits(root), wl.f32_to_bf16_bits(levels)
                   if depth > 1 else np.zeros((0, K, Vd), np.uint16), d2t, K, depth, total, 3)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("kind", ["normal", "integers", "ascending", "descending", "nan_first",
+                                  "nan_later", "inf", "zeros"])
+def test_eagle3_split_rows_heap_order(gpu, oracle, dtype, kind):
+    """Rows split into parts of 4096 values: the root row's ids are the
+    oracle's heap top-k for every k of the register heap, at the edges of a
+    part, with ties, with more candidates than a part stores (ascending rows)
+    and with NaN among the first k values or after them."""
+    import torch
+    import llima_amd
+    rng = np.random.default_rng(41)
+    for k, cols in [(1, 1), (2, 4095), (5, 4096), (5, 4097), (8, 12289), (9, 32001), (13, 8192),
+                    (16, 40007), (5, 262145)]:
+        _say("eagle3 split rows", dtype, kind, k, cols)
+        x = rng.normal(0, 3, cols).astype(np.float32)
+        if kind == "integers":
+            x = rng.integers(-3, 4, cols).astype(np.float32)
+        elif kind in ("ascending", "descending"):
+            x = np.sort(x)[::1 if kind == "ascending" else -1].copy()
+        elif kind == "nan_first":
+            x[min(k - 1, 2)] = np.nan
+        elif kind == "nan_later":
+            x[k::7] = np.nan
+        elif kind == "inf":
+            x[::3], x[1::3] = np.inf, -np.inf
+        elif kind == "zeros":
+            x = np.where(rng.random(cols) < 0.5, 0.0, -0.0).astype(np.float32)
+        xb = wl.f32_to_bf16_bits(x) if dtype == "bf16" else x
+        tree = llima_amd.Eagle3DraftTree(torch.zeros(cols, dtype=torch.int32, device=gpu), topk=k,
+                                         depth=1)
+        pad = torch.cat([torch.zeros(1, dtype=_t(xb, gpu).dtype, device=gpu), _t(xb, gpu)])
+        expect = oracle.topk(xb[None], k)[0][0]
+        assert (_np(tree.begin(_t(xb, gpu))) == expect).all()
+        assert (_np(tree.begin(pad[1:])) == expect).all()          # not 16-byte aligned
+
+
+@pytest.mark.parametrize("K,depth,total,Vd", [(3, 6, 32, 64000), (9, 3, 32, 8191), (10, 4, 20, 12288),
+                                              (16, 2, 32, 4097), (17, 2, 20, 5000), (4, 2, 9, 262145)])
+def test_eagle3_tree_split_rows_shapes(gpu, oracle, K, depth, total, Vd):
+    """Whole trees around the limits of the split rows (k 16, 64 parts)."""
+    _say("eagle3 split tree", K, depth, total, Vd)
+    rng = np.random.default_rng(K * Vd)
+    root = wl.f32_to_bf16_bits(rng.normal(0, 3, Vd).astype(np.float32))
+    levels = wl.f32_to_bf16_bits(rng.normal(0, 3, (depth - 1, K, Vd)).astype(np.float32))
+    d2t = rng.integers(0, 1000, Vd).astype(np.int32)
+    _run_tree(gpu, oracle, root, levels, d2t, K, depth, total, 3)
