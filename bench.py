@@ -172,8 +172,8 @@ def main():
         fin = "lmh_score_finish" if scoring else "lmh_finish"
         if verifying:
             rows, unit_rows = nseq, "sequences/s"
-        kernel_names = (["lmh_packed", fin] if packed else
-                        ["lmh_mfma" if B > 4 else "lmh_rows", fin])
+        kernel_names = (["lmh_tiles" if B > 64 else "lmh_packed", fin] if packed else
+                        ["lmh_tiles" if B > 128 else "lmh_mfma" if B > 4 else "lmh_rows", fin])
         config = {"workload": name, "B": B, "H": H, "V": V,
                   "weight": "bf16 [V, H] packed at load time" if packed else "bf16 [V, H]"}
         data_note = ("synthetic (seeded; one bf16 [%d, %d] weight, %.2f GiB, above the 256 MB "
@@ -275,8 +275,7 @@ def main():
             per = (1 + (depth - 1) * K) * Vd * 2
             alg_bytes = per + Vd * 4 + N * 4 * 3 + N * N * 8
             unit_rows = "trees/s"
-            kernel_names = ["eagle3_begin_kernel", "eagle3_rows_kernel", "eagle3_combine_kernel",
-                            "eagle3_finish_kernel"]
+            kernel_names = ["eagle3_parts_kernel", "eagle3_level_kernel", "eagle3_finish_kernel"]
             config = {"workload": name, "K": K, "depth": depth, "total_tokens": total,
                       "draft_vocab": Vd, "logits_dtype": "bf16",
                       "calls": "begin + %d grow + finish" % (depth - 1)}

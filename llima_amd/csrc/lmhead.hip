@@ -113,17 +113,6 @@ __device__ __forceinline__ void lmh_store_logit(const LmhParams& P, size_t i, fl
         P.out_logits[i] = v;
 }
 
-// Logits i .. i + 3 (i a multiple of 4): one store.
-__device__ __forceinline__ void lmh_store_logits4(const LmhParams& P, size_t i, float4 x) {
-    if (P.logits_bf16) {
-        auto h = [](float v) { return v == v ? __float_as_uint(v) >> 16 : 0x7FC0u; };
-        const uint2 q = make_uint2(h(x.x) | h(x.y) << 16, h(x.z) | h(x.w) << 16);
-        *(uint2*)((uint16_t*)P.out_logits + i) = q;
-    } else {
-        *(float4*)(P.out_logits + i) = x;
-    }
-}
-
 #define LMH_LOG2E 1.44269504088896340736f
 
 // Scoring statistics of one key slot, one logit at a time: m the greatest
@@ -808,6 +797,7 @@ __global__ __launch_bounds__(256) void lmh_tiles(LmhParams P, const uint8_t* wei
         const int n0 = tile * NV, b0 = pass * NM, nb = P.B - b0 < NM ? P.B - b0 : NM;
         uint8_t* const tr = spare + wave * 4096;
         const bool put16 = P.out_logits && P.logits_bf16;    // uniform
+        const bool wide = ((uintptr_t)P.out_logits & 15u) == 0 && V % (P.logits_bf16 ? 8 : 4) == 0;
         // The sums stay in the accumulator registers until their slot reads
         // them (left to the compiler all are moved at once, which spills);
         // an MFMA's result may be read 19 wait states after it.
@@ -837,7 +827,7 @@ __global__ __launch_bounds__(256) void lmh_tiles(LmhParams P, const uint8_t* wei
                         lmh_lds_write(tr + r * 128 + (((k >> 2) ^ (r >> 1 & 7)) << 4) + 8 * g,
                                       make_uint2(h(x[k]) | h(x[k + 1]) << 16, h(x[k + 2]) | h(x[k + 3]) << 16));
                     uint16_t* out = (uint16_t*)P.out_logits + n;
-                    if (V % 8 == 0) {                        // 16-byte pieces, wholly inside or outside
+                    if (wide) {                              // 16-byte pieces, wholly inside or outside
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
                             const int mr = 8 * q + (lane >> 3), ch = lane & 7;
@@ -855,7 +845,7 @@ __global__ __launch_bounds__(256) void lmh_tiles(LmhParams P, const uint8_t* wei
 #pragma unroll
                     for (int k = 0; k < 32; k += 4) {
                         float* o = P.out_logits + (size_t)(b0 + m) * V + n + col(k);
-                        if (row && V % 4 == 0) {
+                        if (row && wide) {
                             if (col(k) < left) *(float4*)o = make_float4(x[k], x[k + 1], x[k + 2], x[k + 3]);
                         } else if (row) {
 #pragma unroll

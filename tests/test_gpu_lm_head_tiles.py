@@ -93,3 +93,31 @@ def test_tiles_ties_nan_and_infinities(gpu, oracle, packed):
     wt = llima_amd.lm_head_pack(wt) if packed else wt
     ids, vals, lg = llima_amd.lm_head_argmax(_t(x, gpu), wt, return_logits=True, logit_dtype="f32")
     assert int(ids[4]) == 0 and float(vals[4]) == -np.inf and bool((lg[4] == -np.inf).all())
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_tiles_logits_output_not_16_byte_aligned(gpu, bf16):
+    """The C entry point writes the same logits at an address that is aligned to
+    its values alone, and nothing beside them."""
+    import torch
+    import llima_amd
+    from llima_amd import _lib
+    _say("lm head tiles unaligned logits", bf16)
+    B, H, V = 130, 256, 520
+    g = torch.Generator(device=gpu).manual_seed(5)
+    x = torch.randn(B, H, device=gpu, generator=g).to(torch.bfloat16)
+    w = llima_amd.lm_head_pack(torch.randn(V, H, device=gpu, generator=g).to(torch.bfloat16))
+    ids, _, lg = llima_amd.lm_head_argmax(x, w, return_logits=True,
+                                          logits_out="bf16" if bf16 else "f32")
+    buf = torch.full((B * V + 2,), 7.0, dtype=lg.dtype, device=gpu)
+    out_ids = torch.empty(B, dtype=torch.int32, device=gpu)
+    L = _lib.lib()
+    ws = torch.empty(L.llima_lm_head_argmax_packed_workspace_bytes(B, H, V), dtype=torch.uint8,
+                     device=gpu)
+    ld = _lib.LLIMA_BF16 | (_lib.LLIMA_LOGITS_OUT_BF16 if bf16 else 0)
+    rc = L.llima_lm_head_argmax_packed(x.data_ptr(), w.data.data_ptr(), B, H, V, 0.0, ld,
+                                       out_ids.data_ptr(), None, buf[1:].data_ptr(), ws.data_ptr(),
+                                       ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(buf[1:-1].reshape(B, V), lg) and torch.equal(out_ids, ids)
+    assert float(buf[0]) == 7.0 and float(buf[-1]) == 7.0
