@@ -126,7 +126,6 @@ struct SampleParams {
     int32_t rank;        // bound_rank of the broadcast top-k (per-row k: computed per row)
     int32_t wide;        // sample_finish_wide ran first: finish only the rows it left pending
     int32_t fsplit;      // sample_finish workgroups per row (> 1: rows without top-k may be split)
-    int32_t mixed;       // per-row top-k: the rows without it take the dense path's kernels
     int32_t rcpw;        // chunks per part of a split row (at most SMP_RCPW)
     int32_t scap;        // values a split row's chunk stages (at most SMP_STG_CAP)
     uint64_t* xstg;      // [B][S][SMP_XSTG] split-row staging beyond the regions
@@ -170,14 +169,6 @@ __device__ __forceinline__ RowCfg load_cfg(const SampleParams& P, int row) {
     r.pen = h > 0 && (r.R != 1.0f || r.alpha != 0.0f || r.beta != 0.0f);
     if (!(r.k > 0 && r.k < P.V)) r.k = 0;
     return r;
-}
-
-// Whether a row takes the dense path's kernels: every row of a batch without
-// top-k, and in a mixed batch (per-row top-k) the rows without it, whose
-// candidates would overflow their regions.  A row at an infinite temperature
-// there stays with sample_finish (the full-row path).
-__device__ __forceinline__ bool dense_row(const SampleParams& P, const RowCfg& c) {
-    return !P.mixed || (!c.greedy && c.k == 0 && c.T < __builtin_inff());
 }
 
 // A row's penalties are applied by the finish, to its candidates only, when
@@ -249,29 +240,6 @@ __device__ __forceinline__ uint32_t pre_slots(const SampleParams& P) {
     return n < SMP_REGION ? n : SMP_REGION;
 }
 
-// Dense path: slots of a row's regions (the dense path's comment says how they
-// are used).
-#define SMP_DSTAT 448                              // chunk max key << 32 | 1 when it holds a finite value
-#define SMP_DBEST 449                              // greedy: key << 32 | ~id of the chunk maximum
-#define SMP_DKEPT 450                              // kept mass strictly above the boundary bin
-#define SMP_DMCNT 451                              // the chunk's members of the boundary bin
-#define SMP_DSWIN 452                              // the chunk's staged top window
-#define SMP_DINFO 456                              // region 0: boundary bin, mass above it, Z
-#define SMP_DMEM 496                               // region 0: boundary members appended
-#define SMP_DMCAP 4096                             // members dense_final ranks (16 per thread)
-#define SMP_DMWG 512                               // members a dense_keep workgroup stages
-
-// A chunk's statistics from its maximum key before / T (km; f32_key(-inf): no
-// value above -inf): the key of the quotient, and whether it is above -inf.
-// l / T is monotone in l, so the largest quotient is the quotient of the
-// largest l, and it rounds to -inf exactly when l <= -T (2^128 - 2^103) (exact
-// in double).
-__device__ __forceinline__ void dense_put_stat(uint64_t* reg, uint32_t km, float T) {
-    const float lm = key_f32(km);
-    const uint32_t any = (double)lm > -(double)T * 3.4028235677973366e38 ? 1u : 0u;
-    reg[SMP_DSTAT] = ((uint64_t)(any ? f32_key(lm / T) : 0u) << 32) | any;
-}
-
 // ================================================================== sweep
 // VEC: rows are 16-byte aligned and V is a multiple of the values per load, so
 // every chunk (also a row's partial last one) is read with 16-byte loads from
@@ -282,8 +250,7 @@ __device__ __forceinline__ void dense_put_stat(uint64_t* reg, uint32_t km, float
 // requested once chunk cc has arrived and before it is processed, so the
 // processing overlaps the next transfer (with every load of the grid issued at
 // once, each chunk completes only when the last of all requests does).
-// MIX: a mixed batch; its dense rows get the chunk statistics dense_stats writes.
-template <typename TL, bool VEC, bool MASK, int SC, bool MIX>
+template <typename TL, bool VEC, bool MASK, int SC>
 __global__ __launch_bounds__(LLIMA_WG) void sample_sweep(SampleParams P) {
     constexpr int EPL = 16 / sizeof(TL);       // values per 16-byte load
     constexpr int NL = 4;                      // 16-byte loads per thread and chunk
@@ -473,21 +440,6 @@ __global__ __launch_bounds__(LLIMA_WG) void sample_sweep(SampleParams P) {
         }
 
         uint64_t* reg = region_of(P, row, chunk);
-        if constexpr (MIX) {
-            if (dense_row(P, c)) {                               // uniform
-                const uint32_t wk = wave_max_u32(lm > NEG_INF ? f32_key(lm) : LLIMA_KEY_NEG_INF);
-                if (lane == 0) xa[cc][wave] = wk;
-                __syncthreads();
-                if (t == 0) {
-                    uint32_t km = 0;
-#pragma unroll
-                    for (int w = 0; w < LLIMA_WAVES; ++w) km = xa[cc][w] > km ? xa[cc][w] : km;
-                    dense_put_stat(reg, km, c.T);
-                    if (chunk == 0) reg[SMP_DMEM] = 0;
-                }
-                continue;
-            }
-        }
         if (c.greedy) {
             // ---- argmax: first index of the maximum (values visited in index order)
             float best = NEG_INF;
@@ -3032,131 +2984,14 @@ __device__ __forceinline__ bool fin_direct(const SampleParams& P, int row, const
 
 // SPLIT: the instantiation launched when rows may be split (P.fsplit > 1); the
 // split code stays out of the other one, whose registers it would crowd.
-// The row's maximum key and whether it has a finite value (nfin, the number of
-// chunks with one) from the chunks' statistics, read
-// by every wave (lane i: chunks i, i + 64, ...) and reduced with DPP.
-__device__ __forceinline__ void dense_row_stats(const SampleParams& P, int row, uint32_t* kmax,
-                                                uint32_t* nfin) {
-    const uint64_t* r0 = region_of(P, (uint32_t)row, 0);
-    uint32_t km = 0, nf = 0;
-    for (int i = (int)lane_id(); i < P.S; i += 64) {
-        const uint64_t v = r0[(size_t)i * SMP_REGION + SMP_DSTAT];
-        const uint32_t k = (uint32_t)(v >> 32);
-        km = k > km ? k : km;
-        nf += (uint32_t)v;
-    }
-    *kmax = wave_max_u32(km);
-    *nfin = wave_sum_u32(nf);
-}
-
-// Dense path: the top-p boundary bin of a row from its chunks' bins, by one
-// workgroup: thread t merges bins 2t and 2t + 1 over the chunks (16-byte loads of up
-// to 32 chunks issued before any is used), then a block scan gives each bin's
-// mass above.
-__device__ __forceinline__ void dense_bound_row(const SampleParams& P, int row, const RowCfg& c,
-                                                BlockScratch& bs) {
-    if (c.greedy || !(c.p < 1.0f)) return;              // uniform: no top-p on this row
-    uint32_t kmax, nfin;
-    dense_row_stats(P, row, &kmax, &nfin);
-    if (nfin == 0) return;
-    const uint32_t t = threadIdx.x;
-    uint64_t* r0 = region_of(P, (uint32_t)row, 0);
-    uint32_t cn0 = 0, cn1 = 0;
-    uint64_t m0 = 0, m1 = 0;
-    if (t < SMP_DBINS / 2) {
-        constexpr int NB = 32;
-        for (int b0 = 0; b0 < P.S; b0 += NB) {
-            llima_u32x4 q[NB];
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const int ci = b0 + i < P.S ? b0 + i : P.S - 1;
-                q[i] = *(const llima_u32x4*)(r0 + (size_t)ci * SMP_REGION + 2u * t);
-            }
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const bool in = b0 + i < P.S;
-                const uint64_t h0 = in ? ((uint64_t)q[i].y << 32) | q[i].x : 0ull;
-                const uint64_t h1 = in ? ((uint64_t)q[i].w << 32) | q[i].z : 0ull;
-                cn0 += (uint32_t)(h0 & 0x3FFFu);
-                m0 += h0 >> 14;
-                cn1 += (uint32_t)(h1 & 0x3FFFu);
-                m1 += h1 >> 14;
-            }
-        }
-    }
-    uint64_t Z;
-    const uint64_t ab = block_excl_scan_u64(m0 + m1, &Z, bs);   // mass above bin 2t
-    const llima_u128 PZ = (llima_u128)frac32(c.p) * Z;
-    const bool q0 = cn0 > 0u && (((llima_u128)ab << 32) < PZ);
-    const bool q1 = cn1 > 0u && (((llima_u128)(ab + m0) << 32) < PZ);
-    const uint32_t qb = block_max_u32(q1 ? 2u * t + 2u : (q0 ? 2u * t + 1u : 0u), bs);
-    const uint32_t ne = cn0 ? 2u * t : (cn1 ? 2u * t + 1u : 0xFFFFFFFFu);
-    const uint32_t top = ~block_max_u32(~ne, bs);               // top non-empty bin
-    const uint32_t bstar = qb ? qb - 1u : top;
-    if ((bstar >> 1) == t) {
-        r0[SMP_DINFO] = bstar;
-        r0[SMP_DINFO + 1] = (bstar & 1u) ? ab + m0 : ab;
-        r0[SMP_DINFO + 2] = Z;
-    }
-    // each chunk's count in b*, so that dense_keep skips the chunks without members
-    for (int i = (int)t; i < P.S; i += LLIMA_WG) {
-        uint64_t* reg = r0 + (size_t)i * SMP_REGION;
-        reg[SMP_DMCNT] = reg[bstar] & 0x3FFFu;
-    }
-    if (!(c.m > 0.0f)) {
-        // Without min-p every value above b* is kept, so each chunk's kept
-        // mass is the sum of its bins before b*: 8 threads per chunk (32
-        // chunks per round), thread part p summing bin pairs p, p + 8, ...
-        // (4 loads in flight), then a reduction over the 8 lanes.
-        const uint32_t part = t & 7u, npairs = (bstar + 1u) >> 1;
-        for (int cb = 0; cb < P.S; cb += LLIMA_WG / 8) {
-            const int ci = cb + (int)(t >> 3);
-            const uint64_t* reg = r0 + (size_t)(ci < P.S ? ci : 0) * SMP_REGION;
-            uint64_t acc = 0;
-            for (uint32_t q0 = part; q0 < npairs; q0 += 32u) {
-                llima_u32x4 h[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t q = q0 + 8u * (uint32_t)k;
-                    h[k] = *(const llima_u32x4*)(reg + 2u * (q < npairs ? q : 0u));
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t q = q0 + 8u * (uint32_t)k;
-                    const uint64_t a = ((uint64_t)h[k].y << 32) | h[k].x, b = ((uint64_t)h[k].w << 32) | h[k].z;
-                    acc += q < npairs ? (a >> 14) + (2u * q + 1u < bstar ? b >> 14 : 0ull) : 0ull;
-                }
-            }
-#pragma unroll
-            for (int sft = 1; sft < 8; sft <<= 1) {
-                const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)acc, sft);
-                const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(acc >> 32), sft);
-                acc += ((uint64_t)hi << 32) | lo;
-            }
-            if (part == 0 && ci < P.S) r0[(size_t)ci * SMP_REGION + SMP_DKEPT] = acc;
-        }
-    }
-}
-
-// MODE: FIN_LEAN; FIN_SPLIT, several workgroups per row (rows without top-k
-// whose regions overflowed are split over them); FIN_MIXED, a mixed batch (the
-// dense rows' workgroups find their boundary bin, beside the other rows'
-// finish).
-enum { FIN_LEAN, FIN_SPLIT, FIN_MIXED };
-template <typename TL, int MODE>
+template <typename TL, bool SPLIT>
 __global__ __launch_bounds__(LLIMA_WG) void sample_finish(SampleParams P) {
     __shared__ FinShared sh;
     FIN_BEGIN();
     const int row = blockIdx.x;
     if (P.wide && P.out_ids[row] != SMP_PENDING) return;     // uniform: finished by the wide kernel
     const RowCfg c = load_cfg(P, row);
-    if constexpr (MODE == FIN_MIXED) {
-        if (dense_row(P, c)) {                                // uniform
-            dense_bound_row(P, row, c, sh.bs);
-            return;
-        }
-    }
-    if constexpr (MODE == FIN_SPLIT) {
+    if constexpr (SPLIT) {
         if (!c.greedy && c.k == 0) {                          // uniform: the row may be split
             const uint32_t kx = split_row(P, row, c, sh);
             if (kx) {
@@ -3605,8 +3440,8 @@ __global__ __launch_bounds__(SMP_WIDE) void sample_finish_wide(SampleParams P) {
 // These rows are selected instead by the workgroups of all their chunks in
 // parallel (one 16 KB chunk per workgroup, the sweep's lane layout), over
 // three reads of the row:
-//   dense_stats  the chunk's maximum key and whether it has a finite value, or
-//                on greedy rows its (key, first id) maximum;
+//   dense_stats  the chunk's maximum key and finite count, or on greedy rows
+//                its (key, first id) maximum;
 //   dense_hist   rows with top-p: the chunk's exact weights counted into
 //                SMP_DBINS value bins of 1/16 nat below the row maximum (bin
 //                floor(16 (xmax - x)), monotone in the key, the last open) as
@@ -3646,6 +3481,15 @@ __global__ __launch_bounds__(SMP_WIDE) void sample_finish_wide(SampleParams P) {
 //   region 0, SMP_DINFO..+2         dense_bound's boundary bin, mass above it, Z
 //   region 0, SMP_DMEM              members appended (a 128-byte line of its
 //                                   own), zeroed by dense_stats
+#define SMP_DSTAT 448                              // chunk max key << 32 | finite count
+#define SMP_DBEST 449                              // greedy: key << 32 | ~id of the chunk maximum
+#define SMP_DKEPT 450                              // kept mass strictly above the boundary bin
+#define SMP_DMCNT 451                              // the chunk's members of the boundary bin
+#define SMP_DSWIN 452                              // the chunk's staged top window
+#define SMP_DINFO 456                              // region 0: boundary bin, mass above it, Z
+#define SMP_DMEM 496                               // region 0: boundary members appended
+#define SMP_DMCAP 4096                             // members dense_final ranks (16 per thread)
+#define SMP_DMWG 512                               // members a dense_keep workgroup stages
 static_assert(SMP_DBINS <= SMP_DSTAT && SMP_DMEM + 16 <= SMP_REGION, "dense region layout");
 static_assert(SMP_DMCAP == 16 * LLIMA_WG, "dense_final holds 16 members per thread");
 
@@ -3762,33 +3606,16 @@ __device__ __forceinline__ void dense_unpack(const SampleParams& P, const RowCfg
                                              const llima_u32x4 (&raw)[DenseGeom<TL>::NL],
                                              const uint32_t* table, float (&x)[DenseGeom<TL>::E]) {
     using G = DenseGeom<TL>;
-    // no test per value for the row's end or the penalties where neither can
-    // apply (uniform; fp32: a second copy for bf16's 32 values per thread does
-    // not fit the 64 registers of eight waves per SIMD)
-    const bool plain = sizeof(TL) == 4 && !c.pen && c0 + G::CHUNK <= P.V;
-    auto bits = [&](const uint32_t (&w4)[4], int e) {
-        if constexpr (sizeof(TL) == 4) return w4[e];
-        else return (e & 1) ? (w4[e >> 1] & 0xFFFF0000u) : (w4[e >> 1] << 16);
-    };
-    if (plain) {
-#pragma unroll
-        for (int j = 0; j < G::NL; ++j) {
-            const uint32_t w4[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-#pragma unroll
-            for (int e = 0; e < G::EPL; ++e) {
-                const float l = __uint_as_float(bits(w4, e));
-                x[j * G::EPL + e] = l == l ? l : -__builtin_inff();
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int j = 0; j < G::NL; ++j) {
         const uint32_t w4[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
         for (int e = 0; e < G::EPL; ++e) {
             const int i = dense_id<TL>(c0, j, e);
-            float l = i < P.V ? __uint_as_float(bits(w4, e)) : -__builtin_inff();
+            uint32_t bits;
+            if constexpr (sizeof(TL) == 4) bits = w4[e];
+            else bits = (e & 1) ? (w4[e >> 1] & 0xFFFF0000u) : (w4[e >> 1] << 16);
+            float l = i < P.V ? __uint_as_float(bits) : -__builtin_inff();
             if (l != l) l = -__builtin_inff();
             const uint32_t cnt = c.pen ? table_count(table, (uint32_t)(i - c0)) : 0u;
             x[j * G::EPL + e] = cnt ? penalize(l, cnt, c) : l;
@@ -3803,6 +3630,22 @@ __device__ __forceinline__ void dense_div(float (&x)[E], const RowCfg& c) {
 #pragma unroll
         for (int i = 0; i < E; ++i) x[i] = x[i] / c.T;
     }
+}
+
+// The row's maximum key and finite count from the chunks' statistics, read
+// by every wave (lane i: chunks i, i + 64, ...) and reduced with DPP.
+__device__ __forceinline__ void dense_row_stats(const SampleParams& P, int row, uint32_t* kmax,
+                                                uint32_t* nfin) {
+    const uint64_t* r0 = region_of(P, (uint32_t)row, 0);
+    uint32_t km = 0, nf = 0;
+    for (int i = (int)lane_id(); i < P.S; i += 64) {
+        const uint64_t v = r0[(size_t)i * SMP_REGION + SMP_DSTAT];
+        const uint32_t k = (uint32_t)(v >> 32);
+        km = k > km ? k : km;
+        nf += (uint32_t)v;
+    }
+    *kmax = wave_max_u32(km);
+    *nfin = wave_sum_u32(nf);
 }
 
 template <typename TL>
@@ -3836,19 +3679,117 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
         best = block_max_u64(best, bs);
         if (threadIdx.x == 0) reg[SMP_DBEST] = best;
     } else {
+        // no division: l / T is monotone in l, so the largest quotient is the
+        // quotient of the largest l, and l / T rounds to -inf exactly when
+        // l <= -T (2^128 - 2^103) (exact in double), so both follow from l
+        const double thr = -(double)c.T * 3.4028235677973366e38;
         float lm = -__builtin_inff();
+        uint32_t nf = 0;
 #pragma unroll
-        for (int i = 0; i < G::E; ++i) lm = __builtin_fmaxf(lm, x[i]);
-        const uint32_t km = block_max_u32(f32_key(lm), bs);
-        if (threadIdx.x == 0) dense_put_stat(reg, km, c.T);
+        for (int i = 0; i < G::E; ++i) {
+            lm = __builtin_fmaxf(lm, x[i]);
+            nf += (double)x[i] > thr ? 1u : 0u;
+        }
+        uint32_t km = f32_key(lm);
+        km = block_max_u32(km, bs);
+        nf = block_sum_u32(nf, bs);
+        if (threadIdx.x == 0) {
+            const float xm = key_f32(km) / c.T;
+            reg[SMP_DSTAT] = ((uint64_t)(nf ? f32_key(xm) : 0u) << 32) | nf;
+        }
     }
     if (chunk == 0 && threadIdx.x == 0) reg[SMP_DMEM] = 0;
 }
 
-// dense_bound_row of every row of a batch without top-k.
+// The top-p boundary bin of each row from its chunks' bins, one workgroup per
+// row: thread t merges bins 2t and 2t + 1 over the chunks (16-byte loads of up
+// to 32 chunks issued before any is used), then a block scan gives each bin's
+// mass above.
 __global__ __launch_bounds__(LLIMA_WG) void dense_bound(SampleParams P) {
     __shared__ BlockScratch bs;
-    dense_bound_row(P, (int)blockIdx.x, load_cfg(P, (int)blockIdx.x), bs);
+    const int row = blockIdx.x;
+    const RowCfg c = load_cfg(P, row);
+    if (c.greedy || !(c.p < 1.0f)) return;              // uniform: no top-p on this row
+    uint32_t kmax, nfin;
+    dense_row_stats(P, row, &kmax, &nfin);
+    if (nfin == 0) return;
+    const uint32_t t = threadIdx.x;
+    uint64_t* r0 = region_of(P, (uint32_t)row, 0);
+    uint32_t cn0 = 0, cn1 = 0;
+    uint64_t m0 = 0, m1 = 0;
+    if (t < SMP_DBINS / 2) {
+        constexpr int NB = 32;
+        for (int b0 = 0; b0 < P.S; b0 += NB) {
+            llima_u32x4 q[NB];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int ci = b0 + i < P.S ? b0 + i : P.S - 1;
+                q[i] = *(const llima_u32x4*)(r0 + (size_t)ci * SMP_REGION + 2u * t);
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const bool in = b0 + i < P.S;
+                const uint64_t h0 = in ? ((uint64_t)q[i].y << 32) | q[i].x : 0ull;
+                const uint64_t h1 = in ? ((uint64_t)q[i].w << 32) | q[i].z : 0ull;
+                cn0 += (uint32_t)(h0 & 0x3FFFu);
+                m0 += h0 >> 14;
+                cn1 += (uint32_t)(h1 & 0x3FFFu);
+                m1 += h1 >> 14;
+            }
+        }
+    }
+    uint64_t Z;
+    const uint64_t ab = block_excl_scan_u64(m0 + m1, &Z, bs);   // mass above bin 2t
+    const llima_u128 PZ = (llima_u128)frac32(c.p) * Z;
+    const bool q0 = cn0 > 0u && (((llima_u128)ab << 32) < PZ);
+    const bool q1 = cn1 > 0u && (((llima_u128)(ab + m0) << 32) < PZ);
+    const uint32_t qb = block_max_u32(q1 ? 2u * t + 2u : (q0 ? 2u * t + 1u : 0u), bs);
+    const uint32_t ne = cn0 ? 2u * t : (cn1 ? 2u * t + 1u : 0xFFFFFFFFu);
+    const uint32_t top = ~block_max_u32(~ne, bs);               // top non-empty bin
+    const uint32_t bstar = qb ? qb - 1u : top;
+    if ((bstar >> 1) == t) {
+        r0[SMP_DINFO] = bstar;
+        r0[SMP_DINFO + 1] = (bstar & 1u) ? ab + m0 : ab;
+        r0[SMP_DINFO + 2] = Z;
+    }
+    // each chunk's count in b*, so that dense_keep skips the chunks without members
+    for (int i = (int)t; i < P.S; i += LLIMA_WG) {
+        uint64_t* reg = r0 + (size_t)i * SMP_REGION;
+        reg[SMP_DMCNT] = reg[bstar] & 0x3FFFu;
+    }
+    if (!(c.m > 0.0f)) {
+        // Without min-p every value above b* is kept, so each chunk's kept
+        // mass is the sum of its bins before b*: 8 threads per chunk (32
+        // chunks per round), thread part p summing bin pairs p, p + 8, ...
+        // (4 loads in flight), then a reduction over the 8 lanes.
+        const uint32_t part = t & 7u, npairs = (bstar + 1u) >> 1;
+        for (int cb = 0; cb < P.S; cb += LLIMA_WG / 8) {
+            const int ci = cb + (int)(t >> 3);
+            const uint64_t* reg = r0 + (size_t)(ci < P.S ? ci : 0) * SMP_REGION;
+            uint64_t acc = 0;
+            for (uint32_t q0 = part; q0 < npairs; q0 += 32u) {
+                llima_u32x4 h[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t q = q0 + 8u * (uint32_t)k;
+                    h[k] = *(const llima_u32x4*)(reg + 2u * (q < npairs ? q : 0u));
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t q = q0 + 8u * (uint32_t)k;
+                    const uint64_t a = ((uint64_t)h[k].y << 32) | h[k].x, b = ((uint64_t)h[k].w << 32) | h[k].z;
+                    acc += q < npairs ? (a >> 14) + (2u * q + 1u < bstar ? b >> 14 : 0ull) : 0ull;
+                }
+            }
+#pragma unroll
+            for (int sft = 1; sft < 8; sft <<= 1) {
+                const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)acc, sft);
+                const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(acc >> 32), sft);
+                acc += ((uint64_t)hi << 32) | lo;
+            }
+            if (part == 0 && ci < P.S) r0[(size_t)ci * SMP_REGION + SMP_DKEPT] = acc;
+        }
+    }
 }
 
 template <typename TL>
@@ -3861,7 +3802,6 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     map_row_chunk(blockIdx.x, (uint32_t)P.B, (uint32_t)P.S, &row, &chunk);
     if (row >= (uint32_t)P.B) return;
     const int c0 = (int)chunk * G::CHUNK;
-    if (P.mixed && !dense_row(P, load_cfg(P, (int)row))) return;   // uniform: before its loads
     int32_t hid[SMP_HBATCH];
     if (P.H_max > 0) dense_hist_ids(P, (int)row, hid);
     llima_u32x4 raw[G::NL];
@@ -3879,31 +3819,16 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     float x[G::E];
     dense_unpack<TL>(P, c, c0, raw, table, x);
     dense_div(x, c);
-    float xmax = key_f32(kmax);
-    // A +inf maximum: its values become 0 and the finite ones a value with
-    // weight 0 in the last bin, so that no value needs a test for it below
-    // (such a row stages no window: the values are not the row's any more).
-    const bool top_inf = xmax == __builtin_inff();      // uniform
-    if (top_inf) {
-#pragma unroll
-        for (int i = 0; i < G::E; ++i)
-            x[i] = x[i] == xmax ? 0.0f : x[i] > -__builtin_inff() ? -1e30f : x[i];
-        xmax = 0.0f;
-    }
-    const WeightSgpr wc;
+    const float xmax = key_f32(kmax);
     uint32_t bin[G::E];                                 // kept for the staging (fp32)
 #pragma unroll
     for (int i = 0; i < G::E; ++i) {
-        const float d0 = x[i] - xmax;                   // -inf: weight 0, bin SMP_DBINS - 1 until the select
-        const float wf = weight_fd(d0, wc);
-        const uint32_t bf = (uint32_t)__builtin_fminf(d0 * -SMP_DBIN_SCALE, (float)(SMP_DBINS - 1));
-        const uint32_t b = x[i] > -__builtin_inff() ? bf : SMP_DBINS + lane;
+        const bool fin = x[i] > -__builtin_inff();
+        const float wf = dense_wf(x[i], xmax);
+        const uint32_t b = fin ? (uint32_t)dense_d16(x[i], xmax) : SMP_DBINS + lane;
         bin[i] = b;
-        // (W << 14) + 1: W below 2^18 and from 2^18 up are exact parts of the float
-        const float hi = __builtin_truncf(wf * 3.814697265625e-06f);
-        const uint32_t lo = (uint32_t)__builtin_fmaf(hi, -262144.0f, wf);
-        atomicAdd((unsigned long long*)&hist[b],
-                  ((unsigned long long)(uint32_t)hi << 32) | (lo << 14 | 1u));
+        // (W << 14) + 1: W 2^14 < 2^51 is an exact integral float
+        atomicAdd((unsigned long long*)&hist[b], (unsigned long long)(wf_u64(wf * 16384.0f) | 1ull));
     }
     __syncthreads();
     uint64_t* reg = region_of(P, row, chunk);
@@ -3917,7 +3842,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     // boundary bin's members from them instead of reading the chunk again.
     // fp32 only: a bf16 thread's 32 values kept live past the binning would
     // not fit the 64 registers of eight waves per SIMD.
-    if (sizeof(TL) != 4 || top_inf) {                    // uniform
+    if constexpr (sizeof(TL) != 4) {
         if (t == 0) reg[SMP_DSWIN] = 0;                  // no window
         return;
     }
@@ -3986,7 +3911,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(sizeof
     if (row >= (uint32_t)P.B) return;
     const int c0 = (int)chunk * G::CHUNK;
     const RowCfg c = load_cfg(P, (int)row);
-    if (c.greedy || !dense_row(P, c)) return;           // dense_final writes greedy rows
+    if (c.greedy) return;                               // dense_final writes greedy rows
     const bool topp = c.p < 1.0f;
     // top-p rows without min-p or a kept-set output need this pass only for
     // the boundary bin's members: chunks without any leave before loading,
@@ -4123,7 +4048,6 @@ __global__ __launch_bounds__(LLIMA_WG) void dense_final(SampleParams P) {
     __shared__ uint64_t drel;
     const int row = blockIdx.x;
     const RowCfg c = load_cfg(P, row);
-    if (!dense_row(P, c)) return;                       // uniform: sample_finish's row
     const uint32_t t = threadIdx.x;
     const int S = P.S;
     uint64_t* r0 = region_of(P, (uint32_t)row, 0);
@@ -4299,43 +4223,28 @@ static void launch_sweep(const SampleParams& P, hipStream_t st) {
     // the history count table (dynamic LDS) only when the sweep penalises
     const size_t cnt_bytes = (P.H_max > 0 && P.eager) ? (size_t)SC * (16 / sizeof(TL)) * 4 * LLIMA_WG / 2 * 4 : 0;
     if (P.bitmask) {
-        if (P.vec_ok) hipLaunchKernelGGL((sample_sweep<TL, true, true, SC, false>), g, b, cnt_bytes, st, P);
-        else hipLaunchKernelGGL((sample_sweep<TL, false, true, SC, false>), g, b, cnt_bytes, st, P);
-    } else if (P.mixed) {
-        if (P.vec_ok) hipLaunchKernelGGL((sample_sweep<TL, true, false, SC, true>), g, b, cnt_bytes, st, P);
-        else hipLaunchKernelGGL((sample_sweep<TL, false, false, SC, true>), g, b, cnt_bytes, st, P);
+        if (P.vec_ok) hipLaunchKernelGGL((sample_sweep<TL, true, true, SC>), g, b, cnt_bytes, st, P);
+        else hipLaunchKernelGGL((sample_sweep<TL, false, true, SC>), g, b, cnt_bytes, st, P);
     } else {
-        if (P.vec_ok) hipLaunchKernelGGL((sample_sweep<TL, true, false, SC, false>), g, b, cnt_bytes, st, P);
-        else hipLaunchKernelGGL((sample_sweep<TL, false, false, SC, false>), g, b, cnt_bytes, st, P);
+        if (P.vec_ok) hipLaunchKernelGGL((sample_sweep<TL, true, false, SC>), g, b, cnt_bytes, st, P);
+        else hipLaunchKernelGGL((sample_sweep<TL, false, false, SC>), g, b, cnt_bytes, st, P);
     }
 }
 
 // The dense path's launches: three reads of the rows by B x S workgroups
-// (dense_hist and the boundary only when some row has top-p), then one
-// workgroup per row.  In a mixed batch the sweep takes the place of
-// dense_stats, and sample_finish, which finishes the rows with top-k, that of
-// dense_bound.
+// (dense_hist and dense_bound only when some row has top-p), then one
+// workgroup per row.
 template <typename TL>
 static void launch_dense(const SampleParams& P, bool topp, hipStream_t st) {
-    const dim3 g((uint32_t)P.B * (uint32_t)P.S), b(LLIMA_WG), rows((uint32_t)P.B);
+    const dim3 g((uint32_t)P.B * (uint32_t)P.S), b(LLIMA_WG);
     const size_t tb = P.H_max > 0 ? (size_t)DenseGeom<TL>::CHUNK / 2 * sizeof(uint32_t) : 0;
-    if (P.mixed) launch_sweep<TL>(P, st);
-    else hipLaunchKernelGGL(dense_stats<TL>, g, b, tb, st, P);
-    if (topp) hipLaunchKernelGGL(dense_hist<TL>, g, b, tb, st, P);
-    if (P.mixed) hipLaunchKernelGGL((sample_finish<TL, FIN_MIXED>), rows, b, 0, st, P);
-    else if (topp) hipLaunchKernelGGL(dense_bound, rows, b, 0, st, P);
+    hipLaunchKernelGGL(dense_stats<TL>, g, b, tb, st, P);
+    if (topp) {
+        hipLaunchKernelGGL(dense_hist<TL>, g, b, tb, st, P);
+        hipLaunchKernelGGL(dense_bound, dim3((uint32_t)P.B), b, 0, st, P);
+    }
     hipLaunchKernelGGL(dense_keep<TL>, g, b, tb, st, P);
-    hipLaunchKernelGGL(dense_final<TL>, rows, b, 0, st, P);
-}
-
-// The sweep and the finish.
-template <typename TL>
-static void launch_two(const SampleParams& P, hipStream_t st) {
-    const dim3 b(LLIMA_WG);
-    launch_sweep<TL>(P, st);
-    if (P.wide) hipLaunchKernelGGL(sample_finish_wide<TL>, dim3(P.B), dim3(SMP_WIDE), 0, st, P);
-    if (P.fsplit > 1) hipLaunchKernelGGL((sample_finish<TL, FIN_SPLIT>), dim3(P.B, P.fsplit), b, 0, st, P);
-    else hipLaunchKernelGGL((sample_finish<TL, FIN_LEAN>), dim3(P.B), b, 0, st, P);
+    hipLaunchKernelGGL(dense_final<TL>, dim3((uint32_t)P.B), b, 0, st, P);
 }
 
 }  // namespace llima
@@ -4426,38 +4335,45 @@ extern "C" int llima_sample(const void* logits, int32_t dtype, int32_t B, int32_
     // takes only the rows it left)
     P.wide = bitmask && !cfg->greedy && !cfg->top_k_rows && !(cfg->top_k > 0 && cfg->top_k < V) &&
              P.S <= SMP_MAX_S;
-    // Per-row top-k: the rows without it take the dense path's kernels beside
-    // the others (mixed batch), unless the scalar top_k in (0, V) is the
-    // caller's word that every row has top-k (a row without then takes the
-    // full-row path: slower, not wrong) and the two lean launches do.
+    // Rows without top-k whose candidates overflow are split over
+    // ceil(S / P.rcpw) finish workgroups in batches that keep the two-launch
+    // path: per-row top-k (rows of either kind), or a mask without top-k.  With
+    // per-row top-k, a scalar top_k in (0, V) is the caller's word that every
+    // row has top-k (a row without then takes the full-row path: slower, not
+    // wrong), and the lean finish is launched.
     const bool rows_may_lack_topk = cfg->top_k_rows && !(cfg->top_k > 0 && cfg->top_k < V);
-    P.mixed = rows_may_lack_topk && !bitmask && !cfg->greedy && P.S <= SMP_MAX_S;
     P.xstg = P.ws + (size_t)B * P.S * SMP_REGION;
     P.rcnt = (uint32_t*)(P.xstg + (size_t)B * P.S * SMP_XSTG);
-    // Masked rows without top-k whose candidates overflow are split over
-    // ceil(S / P.rcpw) finish workgroups.  Chunks per part: three where every
-    // row may be split (the finish's two workgroups per CU still hold all the
-    // parts of 32 rows of 38 chunks), four with per-row top-k.  Staged values
-    // per chunk: about 135 values of a half-masked chunk lie at or above the
-    // row's boundary bin.
+    // Chunks per part: three under a mask (every row of such a batch may be
+    // split, and the finish's two workgroups per CU still hold all the parts
+    // of 32 rows of 38 chunks), four with per-row top-k (the rows with top-k
+    // finish beside the parts; three measured slower there).
     P.rcpw = P.wide ? 3 : SMP_RCPW;
+    // Staged values per chunk: masked rows need more of them for a window that
+    // holds the row's boundary bin (about 135 values of a half-masked chunk lie
+    // at or above it) than unmasked ones, whose extra staging only costs time.
     P.scap = P.wide ? SMP_STG_CAP : 124;
-    P.fsplit = !cfg->greedy && !out_keep && P.S <= SMP_MAX_S &&
-                       (P.wide || (bitmask && rows_may_lack_topk))
+    P.fsplit = (!cfg->greedy && !out_keep && P.S <= SMP_MAX_S && (rows_may_lack_topk || P.wide))
                    ? (P.S + P.rcpw - 1) / P.rcpw : 1;
     // Rows without top-k (and without a mask) take the dense path: their sweep
     // bound would admit nearly every value of ordinary logits.
     const bool dense = !bitmask && !cfg->greedy && !cfg->top_k_rows &&
                        !(cfg->top_k > 0 && cfg->top_k < V) &&
                        (cfg->temperature_rows || cfg->temperature > 0.0f) && P.S <= SMP_MAX_S;
-    if (dense || P.mixed) {
+    if (dense) {
         const bool topp = cfg->top_p_rows || cfg->top_p < 1.0f;
         if (dtype == LLIMA_F32) launch_dense<float>(P, topp, st);
         else launch_dense<uint16_t>(P, topp, st);
     } else if (dtype == LLIMA_F32) {
-        launch_two<float>(P, st);
+        launch_sweep<float>(P, st);
+        if (P.wide) hipLaunchKernelGGL(sample_finish_wide<float>, dim3(B), dim3(SMP_WIDE), 0, st, P);
+        if (P.fsplit > 1) hipLaunchKernelGGL((sample_finish<float, true>), dim3(B, P.fsplit), dim3(LLIMA_WG), 0, st, P);
+        else hipLaunchKernelGGL((sample_finish<float, false>), dim3(B), dim3(LLIMA_WG), 0, st, P);
     } else {
-        launch_two<uint16_t>(P, st);
+        launch_sweep<uint16_t>(P, st);
+        if (P.wide) hipLaunchKernelGGL(sample_finish_wide<uint16_t>, dim3(B), dim3(SMP_WIDE), 0, st, P);
+        if (P.fsplit > 1) hipLaunchKernelGGL((sample_finish<uint16_t, true>), dim3(B, P.fsplit), dim3(LLIMA_WG), 0, st, P);
+        else hipLaunchKernelGGL((sample_finish<uint16_t, false>), dim3(B), dim3(LLIMA_WG), 0, st, P);
     }
     return hipGetLastError() == hipSuccess ? LLIMA_OK : LLIMA_E_HIP;
 }
