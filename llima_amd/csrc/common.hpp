@@ -109,6 +109,35 @@ __device__ __forceinline__ float weight_fd(float d0) {   // d0 = x - xmax
 }
 __device__ __forceinline__ float weight_f(float x, float xmax) { return weight_fd(x - xmax); }
 
+// weight_fd with its constants held in scalar registers (one in a vector
+// register), for kernels that compute a weight per value: a polynomial step is
+// then one instruction, where the compiler otherwise moves each constant into
+// the result register first (five moves per weight).
+struct WeightSgpr {
+    float log2e = 1.44269502162933349609375f, ln2hi = -0.693145751953125f, ln2lo = -1.428606765330187045e-06f;
+    float c7 = 1.98412698412698412698e-04f * LLIMA_TWO36, c6 = 1.38888888888888888889e-03f * LLIMA_TWO36;
+    float c5 = 8.33333333333333333333e-03f * LLIMA_TWO36, c4 = 4.16666666666666666667e-02f * LLIMA_TWO36;
+    float c3 = 1.66666666666666666667e-01f * LLIMA_TWO36, c2 = 0.5f * LLIMA_TWO36, c1 = LLIMA_TWO36;
+    __device__ __forceinline__ WeightSgpr() {
+        asm("" : "+v"(c7));
+        asm("" : "+s"(log2e), "+s"(ln2hi), "+s"(ln2lo), "+s"(c6), "+s"(c5), "+s"(c4), "+s"(c3), "+s"(c2), "+s"(c1));
+    }
+};
+__device__ __forceinline__ float weight_fd(float d0, const WeightSgpr& k) {
+    const float d = __builtin_fmaxf(d0, -26.0f);
+    const float n = __builtin_rintf(d * k.log2e);
+    float r = __builtin_fmaf(n, k.ln2hi, d);
+    r = __builtin_fmaf(n, k.ln2lo, r);
+    float p = __builtin_fmaf(k.c7, r, k.c6);
+    p = __builtin_fmaf(p, r, k.c5);
+    p = __builtin_fmaf(p, r, k.c4);
+    p = __builtin_fmaf(p, r, k.c3);
+    p = __builtin_fmaf(p, r, k.c2);
+    p = __builtin_fmaf(p, r, k.c1);
+    p = __builtin_fmaf(p, r, k.c1);
+    return __builtin_rintf(__builtin_ldexpf(p, (int)n));
+}
+
 // An integral float below 2^52 as uint64 without branches: the part from 2^32
 // up and the rest are each exact (a float's significand has 24 bits).
 __device__ __forceinline__ uint64_t wf_u64(float wf) {

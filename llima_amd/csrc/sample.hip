@@ -3440,8 +3440,8 @@ __global__ __launch_bounds__(SMP_WIDE) void sample_finish_wide(SampleParams P) {
 // These rows are selected instead by the workgroups of all their chunks in
 // parallel (one 16 KB chunk per workgroup, the sweep's lane layout), over
 // three reads of the row:
-//   dense_stats  the chunk's maximum key and finite count, or on greedy rows
-//                its (key, first id) maximum;
+//   dense_stats  the chunk's maximum key and whether it has a finite value, or
+//                on greedy rows its (key, first id) maximum;
 //   dense_hist   rows with top-p: the chunk's exact weights counted into
 //                SMP_DBINS value bins of 1/16 nat below the row maximum (bin
 //                floor(16 (xmax - x)), monotone in the key, the last open) as
@@ -3481,7 +3481,7 @@ __global__ __launch_bounds__(SMP_WIDE) void sample_finish_wide(SampleParams P) {
 //   region 0, SMP_DINFO..+2         dense_bound's boundary bin, mass above it, Z
 //   region 0, SMP_DMEM              members appended (a 128-byte line of its
 //                                   own), zeroed by dense_stats
-#define SMP_DSTAT 448                              // chunk max key << 32 | finite count
+#define SMP_DSTAT 448                              // chunk max key << 32 | 1 when it holds a finite value
 #define SMP_DBEST 449                              // greedy: key << 32 | ~id of the chunk maximum
 #define SMP_DKEPT 450                              // kept mass strictly above the boundary bin
 #define SMP_DMCNT 451                              // the chunk's members of the boundary bin
@@ -3606,16 +3606,33 @@ __device__ __forceinline__ void dense_unpack(const SampleParams& P, const RowCfg
                                              const llima_u32x4 (&raw)[DenseGeom<TL>::NL],
                                              const uint32_t* table, float (&x)[DenseGeom<TL>::E]) {
     using G = DenseGeom<TL>;
+    // no test per value for the row's end or the penalties where neither can
+    // apply (uniform; fp32: a second copy for bf16's 32 values per thread does
+    // not fit the 64 registers of eight waves per SIMD)
+    const bool plain = sizeof(TL) == 4 && !c.pen && c0 + G::CHUNK <= P.V;
+    auto bits = [&](const uint32_t (&w4)[4], int e) {
+        if constexpr (sizeof(TL) == 4) return w4[e];
+        else return (e & 1) ? (w4[e >> 1] & 0xFFFF0000u) : (w4[e >> 1] << 16);
+    };
+    if (plain) {
+#pragma unroll
+        for (int j = 0; j < G::NL; ++j) {
+            const uint32_t w4[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+#pragma unroll
+            for (int e = 0; e < G::EPL; ++e) {
+                const float l = __uint_as_float(bits(w4, e));
+                x[j * G::EPL + e] = l == l ? l : -__builtin_inff();
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < G::NL; ++j) {
         const uint32_t w4[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
 #pragma unroll
         for (int e = 0; e < G::EPL; ++e) {
             const int i = dense_id<TL>(c0, j, e);
-            uint32_t bits;
-            if constexpr (sizeof(TL) == 4) bits = w4[e];
-            else bits = (e & 1) ? (w4[e >> 1] & 0xFFFF0000u) : (w4[e >> 1] << 16);
-            float l = i < P.V ? __uint_as_float(bits) : -__builtin_inff();
+            float l = i < P.V ? __uint_as_float(bits(w4, e)) : -__builtin_inff();
             if (l != l) l = -__builtin_inff();
             const uint32_t cnt = c.pen ? table_count(table, (uint32_t)(i - c0)) : 0u;
             x[j * G::EPL + e] = cnt ? penalize(l, cnt, c) : l;
@@ -3632,7 +3649,8 @@ __device__ __forceinline__ void dense_div(float (&x)[E], const RowCfg& c) {
     }
 }
 
-// The row's maximum key and finite count from the chunks' statistics, read
+// The row's maximum key and whether it has a finite value (nfin, the number of
+// chunks with one) from the chunks' statistics, read
 // by every wave (lane i: chunks i, i + 64, ...) and reduced with DPP.
 __device__ __forceinline__ void dense_row_stats(const SampleParams& P, int row, uint32_t* kmax,
                                                 uint32_t* nfin) {
@@ -3684,18 +3702,14 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
         // l <= -T (2^128 - 2^103) (exact in double), so both follow from l
         const double thr = -(double)c.T * 3.4028235677973366e38;
         float lm = -__builtin_inff();
-        uint32_t nf = 0;
 #pragma unroll
-        for (int i = 0; i < G::E; ++i) {
-            lm = __builtin_fmaxf(lm, x[i]);
-            nf += (double)x[i] > thr ? 1u : 0u;
-        }
+        for (int i = 0; i < G::E; ++i) lm = __builtin_fmaxf(lm, x[i]);
         uint32_t km = f32_key(lm);
         km = block_max_u32(km, bs);
-        nf = block_sum_u32(nf, bs);
         if (threadIdx.x == 0) {
-            const float xm = key_f32(km) / c.T;
-            reg[SMP_DSTAT] = ((uint64_t)(nf ? f32_key(xm) : 0u) << 32) | nf;
+            lm = key_f32(km);
+            const uint32_t any = (double)lm > thr ? 1u : 0u;   // some l / T above -inf
+            reg[SMP_DSTAT] = ((uint64_t)(any ? f32_key(lm / c.T) : 0u) << 32) | any;
         }
     }
     if (chunk == 0 && threadIdx.x == 0) reg[SMP_DMEM] = 0;
@@ -3792,6 +3806,12 @@ __global__ __launch_bounds__(LLIMA_WG) void dense_bound(SampleParams P) {
     }
 }
 
+// 28 vector instructions per binned value: constants in scalar registers, no
+// test for the row's end, the penalties or an infinite maximum per value (41
+// with them: 19.0 us for 64 rows of 128256 fp32 values, now 17.4; dense_stats,
+// which no longer counts the finite values, 9.3 -> 7.7).  A workgroup's data
+// arrives 2.8 to 8.4 us after the first workgroup starts; then unpacking takes
+// 0.6 us, binning 1.8, the window 0.5 and the staging 1.3.
 template <typename TL>
 __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))) void dense_hist(SampleParams P) {
     using G = DenseGeom<TL>;
@@ -3819,16 +3839,31 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     float x[G::E];
     dense_unpack<TL>(P, c, c0, raw, table, x);
     dense_div(x, c);
-    const float xmax = key_f32(kmax);
+    float xmax = key_f32(kmax);
+    // A +inf maximum: its values become 0 and the finite ones a value with
+    // weight 0 in the last bin, so that no value needs a test for it below
+    // (such a row stages no window: the values are not the row's any more).
+    const bool top_inf = xmax == __builtin_inff();      // uniform
+    if (top_inf) {
+#pragma unroll
+        for (int i = 0; i < G::E; ++i)
+            x[i] = x[i] == xmax ? 0.0f : x[i] > -__builtin_inff() ? -1e30f : x[i];
+        xmax = 0.0f;
+    }
+    const WeightSgpr wc;
     uint32_t bin[G::E];                                 // kept for the staging (fp32)
 #pragma unroll
     for (int i = 0; i < G::E; ++i) {
-        const bool fin = x[i] > -__builtin_inff();
-        const float wf = dense_wf(x[i], xmax);
-        const uint32_t b = fin ? (uint32_t)dense_d16(x[i], xmax) : SMP_DBINS + lane;
+        const float d0 = x[i] - xmax;                   // -inf: weight 0, bin SMP_DBINS - 1 until the select
+        const float wf = weight_fd(d0, wc);
+        const uint32_t bf = (uint32_t)__builtin_fminf(d0 * -SMP_DBIN_SCALE, (float)(SMP_DBINS - 1));
+        const uint32_t b = x[i] > -__builtin_inff() ? bf : SMP_DBINS + lane;
         bin[i] = b;
-        // (W << 14) + 1: W 2^14 < 2^51 is an exact integral float
-        atomicAdd((unsigned long long*)&hist[b], (unsigned long long)(wf_u64(wf * 16384.0f) | 1ull));
+        // (W << 14) + 1: W below 2^18 and from 2^18 up are exact parts of the float
+        const float hi = __builtin_truncf(wf * 3.814697265625e-06f);
+        const uint32_t lo = (uint32_t)__builtin_fmaf(hi, -262144.0f, wf);
+        atomicAdd((unsigned long long*)&hist[b],
+                  ((unsigned long long)(uint32_t)hi << 32) | (lo << 14 | 1u));
     }
     __syncthreads();
     uint64_t* reg = region_of(P, row, chunk);
@@ -3842,7 +3877,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     // boundary bin's members from them instead of reading the chunk again.
     // fp32 only: a bf16 thread's 32 values kept live past the binning would
     // not fit the 64 registers of eight waves per SIMD.
-    if constexpr (sizeof(TL) != 4) {
+    if (sizeof(TL) != 4 || top_inf) {                    // uniform
         if (t == 0) reg[SMP_DSWIN] = 0;                  // no window
         return;
     }
