@@ -3700,6 +3700,13 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
         // no division: l / T is monotone in l, so the largest quotient is the
         // quotient of the largest l, and l / T rounds to -inf exactly when
         // l <= -T (2^128 - 2^103) (exact in double), so both follow from l
+        // (an infinite T, which a row may have: a finite l gives 0 and an
+        // infinite one NaN, which is no value)
+        if (c.T == __builtin_inff()) {                  // uniform
+#pragma unroll
+            for (int i = 0; i < G::E; ++i)
+                x[i] = __builtin_fabsf(x[i]) < __builtin_inff() ? x[i] : -__builtin_inff();
+        }
         const double thr = -(double)c.T * 3.4028235677973366e38;
         float lm = -__builtin_inff();
 #pragma unroll
@@ -3760,7 +3767,9 @@ __global__ __launch_bounds__(LLIMA_WG) void dense_bound(SampleParams P) {
     const uint32_t qb = block_max_u32(q1 ? 2u * t + 2u : (q0 ? 2u * t + 1u : 0u), bs);
     const uint32_t ne = cn0 ? 2u * t : (cn1 ? 2u * t + 1u : 0xFFFFFFFFu);
     const uint32_t top = ~block_max_u32(~ne, bs);               // top non-empty bin
-    const uint32_t bstar = qb ? qb - 1u : top;
+    // top is a bin: the row has a value above -inf, which dense_hist counted
+    // (without one it would be 0xFFFFFFFF, which indexes nothing)
+    const uint32_t bstar = qb ? qb - 1u : top < SMP_DBINS ? top : SMP_DBINS - 1u;
     if ((bstar >> 1) == t) {
         r0[SMP_DINFO] = bstar;
         r0[SMP_DINFO + 1] = (bstar & 1u) ? ab + m0 : ab;
