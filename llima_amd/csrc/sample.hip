@@ -3702,15 +3702,16 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
         // l <= -T (2^128 - 2^103) (exact in double), so both follow from l
         // (an infinite T, which a row may have: a finite l gives 0 and an
         // infinite one NaN, which is no value)
-        if (c.T == __builtin_inff()) {                  // uniform
-#pragma unroll
-            for (int i = 0; i < G::E; ++i)
-                x[i] = __builtin_fabsf(x[i]) < __builtin_inff() ? x[i] : -__builtin_inff();
-        }
         const double thr = -(double)c.T * 3.4028235677973366e38;
         float lm = -__builtin_inff();
+        if (c.T < __builtin_inff()) {                   // uniform
 #pragma unroll
-        for (int i = 0; i < G::E; ++i) lm = __builtin_fmaxf(lm, x[i]);
+            for (int i = 0; i < G::E; ++i) lm = __builtin_fmaxf(lm, x[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < G::E; ++i)
+                lm = __builtin_fmaxf(lm, x[i] < __builtin_inff() ? x[i] : -__builtin_inff());
+        }
         uint32_t km = f32_key(lm);
         km = block_max_u32(km, bs);
         if (threadIdx.x == 0) {
