@@ -3852,7 +3852,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     float xmax = key_f32(kmax);
     // A +inf maximum: its values become 0 and the finite ones a value with
     // weight 0 in the last bin, so that no value needs a test for it below
-    // (such a row stages no window: the values are not the row's any more).
+    // (the staging puts the infinities back and leaves the last bin out).
     const bool top_inf = xmax == __builtin_inff();      // uniform
     if (top_inf) {
 #pragma unroll
@@ -3887,7 +3887,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
     // boundary bin's members from them instead of reading the chunk again.
     // fp32 only: a bf16 thread's 32 values kept live past the binning would
     // not fit the 64 registers of eight waves per SIMD.
-    if (sizeof(TL) != 4 || top_inf) {                    // uniform
+    if constexpr (sizeof(TL) != 4) {
         if (t == 0) reg[SMP_DSWIN] = 0;                  // no window
         return;
     }
@@ -3899,6 +3899,8 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
 #pragma unroll
     for (int i = 0; i < BPL; ++i) {
         bc[i] = (uint32_t)(hist[BPL * lane + i] & 0x3FFFu);
+        // below a +inf maximum the last bin, all its finite values, never fits
+        if (i == BPL - 1) bc[i] = top_inf && lane == 63 ? SMP_DSTG + 1u : bc[i];
         lsum += bc[i];
     }
     const uint32_t cum = wave_incl_scan_u32(lsum);
@@ -3936,7 +3938,7 @@ __global__ __launch_bounds__(LLIMA_WG) __attribute__((amdgpu_waves_per_eu(8, 8))
                 for (int e = 0; e < G::EPL; ++e)
                     if ((sm >> (j * G::EPL + e)) & 1u) {
                         if (base < SMP_DSTG)                 // always: the window's count
-                            dst[base] = ((uint64_t)f32_key(x[j * G::EPL + e]) << 32) |
+                            dst[base] = ((uint64_t)f32_key(top_inf ? __builtin_inff() : x[j * G::EPL + e]) << 32) |
                                         (uint32_t)dense_id<TL>(c0, j, e);
                         ++base;
                     }

@@ -35,3 +35,25 @@ def test_dense_infinite_temperature(gpu, oracle, dtype, V, keep):
     for _ in range(2):
         _sample_both(gpu, oracle, x if dtype == "f32" else wl.f32_to_bf16_bits(x),
                      rng.random(B).astype(np.float32), None, cfg_rows=rows, want_keep=keep)
+
+
+@pytest.mark.parametrize("keep", [False, True])
+@pytest.mark.parametrize("V", [40, 4096, 12300])
+def test_dense_infinite_maximum(gpu, oracle, V, keep):
+    """Rows whose maximum is +inf: 1, 64 and 65 infinities in one chunk (a
+    window stages at most 64 values), spread over the chunks, all of a chunk's
+    other values few enough to fit beside them, and every value infinite."""
+    _say("sample dense infinite maximum", V, keep)
+    rng = np.random.default_rng(V)
+    B = 7
+    x = (rng.standard_normal((B, V), dtype=np.float32) * np.float32(3.0)).astype(np.float32)
+    for b, n in ((0, 1), (1, 64), (2, 65)):
+        x[b, rng.permutation(min(V, 4096))[:n]] = np.inf
+    x[3, ::17] = np.inf
+    x[4] = -np.inf
+    x[4, :20] = 1.0
+    x[4, 5] = np.inf
+    x[5] = np.inf
+    for p in (0.3, 0.9):
+        _sample_both(gpu, oracle, x, rng.random(B).astype(np.float32),
+                     dict(temperature=0.8, top_p=p), want_keep=keep)
