@@ -123,7 +123,8 @@ class Workspace:
 def _stream(device) -> int:
     # the handle of torch.cuda.current_stream(device) without the Stream object
     # around it (0.1 us a call against 1.9 us)
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    i = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
 
 
 class _TargetCheck:
