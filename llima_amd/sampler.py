@@ -127,6 +127,13 @@ def _stream(device) -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
 
 
+def _capturing(device) -> bool:
+    if device.index == torch.cuda.current_device():     # no context manager in the usual case
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class _TargetCheck:
     """The range check of device-resident scoring targets: begun before the
     scoring kernels are launched and waited for after, so that the wait is for
@@ -135,6 +142,10 @@ class _TargetCheck:
     until the next call: about 40 us a call)."""
 
     def __init__(self, tg: torch.Tensor):
+        # the wait cannot be captured: refused before anything is recorded (a
+        # captured event would spoil the pinned allocator for the process)
+        if _capturing(tg.device):
+            raise RuntimeError("scoring checks its targets on the host and cannot be captured")
         self.host = torch.empty(tg.shape, dtype=torch.int32, pin_memory=True)
         self.host.copy_(tg, non_blocking=True)
         self.done = torch.cuda.Event()
