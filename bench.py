@@ -239,7 +239,7 @@ def main():
         else:
             K, depth, total, Vd = w["K"], w["depth"], w["total"], w["root"].shape[0]
             d2t = torch.from_numpy(w["d2t"]).to(dev)
-            nb = L.llima_eagle3_tree_bytes(K, depth)
+            nb = L.llima_eagle3_tree_split_bytes(K, depth, Vd)
             state = torch.empty(nb, dtype=torch.uint8, device=dev)
             roots = [torch.from_numpy(w["root"].view(np.int16)).to(dev).view(torch.bfloat16)]
             levs = [torch.from_numpy(w["levels"].view(np.int16)).to(dev).view(torch.bfloat16)]

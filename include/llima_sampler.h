@@ -447,8 +447,13 @@ int llima_topk(const void* x, int32_t dtype, int32_t rows, int32_t cols, int64_t
  *           out_position_ids [N], out_retrieve [N][N] (leaf paths from the
  *           root, -1 padded), out_dims [2] = {leaf paths, columns used}.
  * log-softmax uses exp and log rounded once from double (the correctly rounded
- * values; the reference's C library expf/logf agree on all but rare arguments). */
+ * values; the reference's C library expf/logf agree on all but rare arguments).
+ * A `tree` of llima_eagle3_tree_split_bytes(K, depth, Vd) bytes (8-byte aligned)
+ * also has room for the candidates of rows split over several workgroups: the
+ * same results in about three quarters of the time at K = 5, Vd = 32000 (82 KB more;
+ * nothing more where rows are not split, K > 16 or Vd > 262144). */
 size_t llima_eagle3_tree_bytes(int32_t K, int32_t depth);
+size_t llima_eagle3_tree_split_bytes(int32_t K, int32_t depth, int32_t Vd);
 int llima_eagle3_tree_begin(const void* logits, int32_t dtype, int32_t Vd, const int32_t* d2t,
                             int32_t K, int32_t depth, void* tree, size_t tree_bytes,
                             int32_t* out_input_ids, void* stream);

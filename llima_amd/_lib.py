@@ -82,6 +82,7 @@ SIGNATURES = {
                                                         _i32, _vp, _vp, _sz, _vp]),
     "llima_topk": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i64, _i32, _vp, _vp, _vp]),
     "llima_eagle3_tree_bytes": (_sz, [_i32, _i32]),
+    "llima_eagle3_tree_split_bytes": (_sz, [_i32, _i32, _i32]),
     "llima_eagle3_tree_begin": (ctypes.c_int, [_vp, _i32, _i32, _vp, _i32, _i32, _vp, _sz, _vp,
                                                _vp]),
     "llima_eagle3_tree_grow": (ctypes.c_int, [_vp, _i32, _i32, _i64, _vp, _i32, _i32, _i32, _vp,

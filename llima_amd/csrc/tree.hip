@@ -50,7 +50,8 @@ namespace llima {
 // ------------------------------------------------------------------ tree state layout
 // A caller-owned device buffer that persists from begin to finish: the current
 // level's scores, the parent groups, every node's score and token, the draft
-// attention mask, and the per-row top-k of the level being grown.
+// attention mask, and the per-row top-k of the level being grown (total bytes);
+// past them, in a buffer that has room, the candidates of rows split into parts.
 struct TreeLayout {
     size_t score, parent, node_score, node_tok, mask, row_idx, row_val, cand, total;
 };
@@ -72,8 +73,7 @@ __host__ __device__ inline TreeLayout tree_layout(int K, int depth) {
     L.mask = tree_take(&o, 4 * (size_t)K * K * depth);
     L.row_idx = tree_take(&o, 4 * (size_t)K * K);
     L.row_val = tree_take(&o, 4 * (size_t)K * K);
-    L.cand = tree_take(&o, K <= TK_PART_K ? 8 * (size_t)K * TK_PARTS * TK_PSLOTS : 0);
-    L.total = o;
+    L.total = L.cand = o;
     return L;
 }
 
@@ -882,7 +882,7 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
         off += w < wave ? wcnt[w] : 0u;
         total += wcnt[w];
     }
-    uint64_t* slots = st<uint64_t>(P, L.cand) + ((size_t)row * TK_PARTS + part) * TK_PSLOTS;
+    uint64_t* slots = st<uint64_t>(P, L.cand) + ((size_t)row * P.parts + part) * TK_PSLOTS;
 #pragma unroll
     for (int e = 0; e < TK_VPT; ++e)
         if ((cmask >> e) & 1u) {
@@ -903,7 +903,7 @@ __device__ __forceinline__ void parts_replay(const TreeParams& P, const TreeLayo
     auto load = [&](int i) {                                // the row's value i
         return P.bf16 ? tk_load<uint16_t>((const uint16_t*)P.x + r0, i) : tk_load<float>((const float*)P.x + r0, i);
     };
-    const uint64_t* slots = st<uint64_t>(P, L.cand) + (size_t)row * TK_PARTS * TK_PSLOTS;
+    const uint64_t* slots = st<uint64_t>(P, L.cand) + (size_t)row * P.parts * TK_PSLOTS;
     // the first 64 candidates of TK_PSTAGE parts, requested together
     auto fetch = [&](int p0) {
         uint64_t c[TK_PSTAGE];
@@ -1296,11 +1296,24 @@ static bool tree_dims_ok(int32_t K, int32_t depth) {
     return nodes <= TREE_MAX_NODES && (int64_t)K * K * (depth > 1 ? depth - 1 : 1) <= 16384;
 }
 
-// Parts per row when a level's rows are split (0 when they are not: k past the
-// register heap, or more values than TK_PARTS parts hold).
+// Parts per row when a level's rows can be split (0 when they cannot: k past
+// the register heap, or more values than TK_PARTS parts hold), and the bytes of
+// a state that holds the candidates of K such rows.
 static int32_t tree_parts(int32_t K, int32_t Vd) {
-    const int32_t n = (Vd + TK_PART - 1) / TK_PART;
+    const int32_t n = Vd > 0 ? (Vd - 1) / TK_PART + 1 : 0;
     return K <= TK_PART_K && n <= TK_PARTS ? n : 0;
+}
+
+static size_t tree_split_bytes(int32_t K, int32_t depth, int32_t Vd) {
+    return tree_layout(K, depth).total + sizeof(uint64_t) * (size_t)K * tree_parts(K, Vd) * TK_PSLOTS;
+}
+
+// Parts per row of a call: 0 also when the state has no room for the
+// candidates, or is not aligned for their 8-byte slots (its own values are 4
+// bytes wide), so that the state need not be larger than the tree.
+static int32_t tree_call_parts(int32_t K, int32_t depth, int32_t Vd, const void* tree,
+                               size_t tree_bytes) {
+    return tree_bytes >= tree_split_bytes(K, depth, Vd) && (uintptr_t)tree % 8 == 0 ? tree_parts(K, Vd) : 0;
 }
 
 // A level's two kernels over split rows: the parts of `rows` rows, then the
@@ -1359,6 +1372,11 @@ extern "C" size_t llima_eagle3_tree_bytes(int32_t K, int32_t depth) {
     return tree_layout(K, depth).total;
 }
 
+extern "C" size_t llima_eagle3_tree_split_bytes(int32_t K, int32_t depth, int32_t Vd) {
+    if (!tree_dims_ok(K, depth)) return 0;
+    return tree_split_bytes(K, depth, Vd);
+}
+
 extern "C" int llima_eagle3_tree_begin(const void* logits, int32_t dtype, int32_t Vd,
                                        const int32_t* d2t, int32_t K, int32_t depth, void* tree,
                                        size_t tree_bytes, int32_t* out_input_ids, void* stream) {
@@ -1369,7 +1387,7 @@ extern "C" int llima_eagle3_tree_begin(const void* logits, int32_t dtype, int32_
     P.x = logits; P.cols = Vd; P.k = K; P.d2t = d2t; P.state = (char*)tree;
     P.K = K; P.depth = depth; P.out_inputs = out_input_ids;
     P.vec = rows_vec(logits, Vd, dtype);
-    P.parts = tree_parts(K, Vd);
+    P.parts = tree_call_parts(K, depth, Vd, tree, tree_bytes);
     P.bf16 = dtype == LLIMA_BF16;
     hipStream_t st = (hipStream_t)stream;
     if (P.parts) launch_parts(P, 1, st);
@@ -1395,7 +1413,7 @@ extern "C" int llima_eagle3_tree_grow(const void* logits, int32_t dtype, int32_t
     P.state = (char*)tree; P.K = K; P.depth = depth; P.level = level;
     P.out_inputs = out_input_ids; P.out_prow = out_parent_rows; P.out_mask = out_mask;
     P.vec = rows_vec(logits, row_stride, dtype);
-    P.parts = tree_parts(K, Vd);
+    P.parts = tree_call_parts(K, depth, Vd, tree, tree_bytes);
     P.bf16 = dtype == LLIMA_BF16;
     hipStream_t st = (hipStream_t)stream;
     if (P.parts) {

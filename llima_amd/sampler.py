@@ -846,7 +846,8 @@ class Eagle3DraftTree:
         self.d2t = d2t.to(dtype=torch.int32).contiguous()
         _on_gpu(self.d2t)
         self.K, self.depth = int(topk), int(depth)
-        nb = lib().llima_eagle3_tree_bytes(self.K, self.depth)
+        # with room for the candidates of rows split over several workgroups
+        nb = lib().llima_eagle3_tree_split_bytes(self.K, self.depth, self.d2t.numel())
         if nb == 0:
             raise ValueError("topk must be 1..32 and depth 1..16 (at most 16384 nodes)")
         self.dev = self.d2t.device

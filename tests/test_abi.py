@@ -103,6 +103,14 @@ def test_host_only_entry_points():
     assert L.llima_eagle3_tree_grow(p, 1, 32000, 32000, p, 5, 4, 4, p, tb, p, p, p, None) == -1
     assert L.llima_eagle3_tree_finish(p, tb, 5, 4, 33, 0, p, p, p, p, p, None) == -1
     assert L.llima_eagle3_tree_finish(p, tb, 2, 2, 7, 0, p, p, p, p, p, None) == -1  # > nodes
+    # the state of a tree alone stays small; with it, 2 KB of candidates per row and
+    # part of 4096 ids where rows are split (K <= 16, at most 64 parts)
+    assert tb == 2560
+    for K, Vd, parts in ((5, 32000, 8), (5, 4096, 1), (5, 4097, 2), (16, 262144, 64), (5, 262145, 0),
+                         (17, 32000, 0), (5, 2**31 - 1, 0), (5, 0, 0)):
+        assert (L.llima_eagle3_tree_split_bytes(K, 4, Vd) ==
+                L.llima_eagle3_tree_bytes(K, 4) + 2048 * K * parts), (K, Vd)
+    assert L.llima_eagle3_tree_split_bytes(0, 4, 32000) == 0
     # stop check: a vocabulary and a stop mask are required; B = 0 launches nothing
     assert L.llima_stop_check(p, None, 1, 4, None, 100, None, p, None, None) == -1
     assert L.llima_stop_check(p, None, 1, 4, p, 0, None, p, None, None) == -1

@@ -179,3 +179,43 @@ def test_eagle3_tree_split_rows_shapes(gpu, oracle, K, depth, total, Vd):
     levels = wl.f32_to_bf16_bits(rng.normal(0, 3, (depth - 1, K, Vd)).astype(np.float32))
     d2t = rng.integers(0, 1000, Vd).astype(np.int32)
     _run_tree(gpu, oracle, root, levels, d2t, K, depth, total, 3)
+
+
+def test_eagle3_tree_state_sizes(gpu, oracle):
+    """A state of llima_eagle3_tree_bytes (no room for split rows' candidates),
+    one byte short of room, exactly large enough, and one that is only 4-byte
+    aligned give the same tree, and nothing is written past their end."""
+    import torch
+    from llima_amd._lib import LLIMA_BF16, check, lib
+    L = lib()
+    rng = np.random.default_rng(9)
+    K, depth, total, Vd = 5, 3, 12, 9001
+    root = wl.f32_to_bf16_bits(rng.normal(0, 3, Vd).astype(np.float32))
+    levels = wl.f32_to_bf16_bits(rng.normal(0, 3, (depth - 1, K, Vd)).astype(np.float32))
+    d2t = rng.integers(0, 1000, Vd).astype(np.int32)
+    e = oracle.eagle3_tree(root, levels, d2t, K, depth, total, 3, cr=True)
+    xr, xl, d2 = _t(root, gpu), _t(levels, gpu), _t(d2t, gpu)
+    small, split = L.llima_eagle3_tree_bytes(K, depth), L.llima_eagle3_tree_split_bytes(K, depth, Vd)
+    N, sp = total + 1, torch.cuda.current_stream(gpu).cuda_stream
+    for nb, off in ((small, 0), (split - 1, 0), (split, 0), (split, 4)):
+        _say("eagle3 tree state", nb, off)
+        buf = torch.full((split + 64,), 0xAB, dtype=torch.uint8, device=gpu)
+        state = buf[off:].data_ptr()
+        i32 = lambda *s: torch.empty(s, dtype=torch.int32, device=gpu)
+        ids, prow, tok, pos, ret, dims = i32(K), i32(K), i32(N), i32(N), i32(N, N), i32(2)
+        mask = torch.empty(K * K * depth, device=gpu)
+        tmask = torch.empty(N, N, device=gpu)
+        check(L.llima_eagle3_tree_begin(xr.data_ptr(), LLIMA_BF16, Vd, d2.data_ptr(), K, depth, state,
+                                        nb, ids.data_ptr(), sp), "begin")
+        assert (_np(ids) == e["inputs"][0]).all()
+        for lv in range(1, depth):
+            check(L.llima_eagle3_tree_grow(xl[lv - 1].data_ptr(), LLIMA_BF16, Vd, Vd, d2.data_ptr(), K,
+                                           depth, lv, state, nb, ids.data_ptr(), prow.data_ptr(),
+                                           mask.data_ptr(), sp), "grow")
+            assert (_np(ids) == e["inputs"][lv]).all() and (_np(prow) == e["parent_rows"][lv - 1]).all()
+        check(L.llima_eagle3_tree_finish(state, nb, K, depth, total, 3, tok.data_ptr(), tmask.data_ptr(),
+                                         pos.data_ptr(), ret.data_ptr(), dims.data_ptr(), sp), "finish")
+        assert (_np(tok) == e["tokens"]).all() and (_np(tmask) == e["tree_mask"]).all()
+        # rows are not split in the smaller states: the candidate slots stay as they were
+        end = off + (split if nb == split and off == 0 else small)
+        assert bool((buf[end:] == 0xAB).all())
