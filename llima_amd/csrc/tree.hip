@@ -810,8 +810,7 @@ __device__ __forceinline__ void tk_list_merge(uint32_t (&a)[N], const uint32_t (
 // kernel replays each row's parts in order, a wavefront per row.  One
 // workgroup per row instead runs ~900 vector instructions per thread on one
 // CU.  A part with more of them than slots (ascending values) says so in its
-// count, and its values are replayed one by one, as are all values of a row
-// with a NaN among its first k.
+// count, and its values are replayed one by one.
 template <typename TL, int KC>
 __global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
     constexpr int NQ = TK_VPT * (int)sizeof(TL) / 16;
@@ -916,26 +915,64 @@ __device__ __forceinline__ void parts_replay(const TreeParams& P, const TreeLayo
         for (int i = 0; i < TK_PSTAGE; ++i) stage[i][lane] = c[i];
     };
     const uint32_t pn = lane < P.parts ? (uint32_t)slots[(size_t)lane * TK_PSLOTS] : 0u;
+    // The values that exceed the root's key, in id order: insert takes a key and
+    // its id and returns the new root's key.  One copy of the loop per heap: the
+    // code runs once per row, so its length is instruction fetch (unrolled over
+    // the parts it took 113 us).
+    auto replay = [&](uint32_t root, auto insert) {
+#pragma unroll 1
+        for (int p = 0; p < P.parts; ++p) {
+            if (p % TK_PSTAGE == 0) fetch(p);
+            const uint32_t stored = (uint32_t)__builtin_amdgcn_readlane((int)pn, p);
+            const bool raw = stored > TK_PSLOTS - 1;        // not all stored: the part's values
+            const int base = p * TK_PART;
+            const int n = !raw ? (int)stored : P.cols - base < TK_PART ? P.cols - base : TK_PART;
+#pragma unroll 1
+            for (int g = 0; g < n; g += 64) {               // 64 values in id order (key 0: none)
+                const int e = g + lane;
+                uint32_t x = 0u;
+                int32_t xj = base + e;
+                if (raw) {
+                    const float f = e < n ? load(base + e) : __builtin_nanf("");
+                    x = xj >= KC && f == f ? f32_key(f) : 0u;
+                } else {
+                    const uint64_t v = g == 0 ? stage[p % TK_PSTAGE][lane]
+                                              : slots[(size_t)p * TK_PSLOTS + 1 + (e < n ? e : g)];
+                    x = e < n ? (uint32_t)(v >> 32) : 0u;
+                    xj = (int32_t)(uint32_t)v;
+                }
+                uint64_t m = ballot(x > root);
+                while (m) {
+                    const int Ln = __builtin_ctzll(m);
+                    root = insert((uint32_t)__builtin_amdgcn_readlane((int)x, Ln),
+                                  __builtin_amdgcn_readlane(xj, Ln));
+                    m = ballot(x > root) & (Ln == 63 ? 0ull : (~0ull << (Ln + 1)));
+                }
+            }
+        }
+    };
     const float f0 = lane < KC ? load(lane) : 0.0f;
-    const bool nan0 = ballot(f0 != f0) != 0ull;             // uniform
-    if (nan0) {                                             // NaNs in the heap: float compares
+    int32_t ri = 0;                                         // lane a: the id of place a
+    if (ballot(f0 != f0)) {                                 // uniform: NaNs in the heap
+        // Float compares, under which a NaN never moves and ends the sift above
+        // it.  The slots the sift reaches from the root are a heap of their own
+        // and the others hold at most the rest of the first k values, so at most
+        // k - 1 values seen exceed the root: the values that do are candidates
+        // here too.  A NaN root lets none in.
         float hv = f0;
         int32_t hi = lane;
         for (int j = KC / 2 - 1; j >= 0; --j) heap_sift(hv, hi, j, KC);
-        float root = rdl_f(hv, 0);
-        for (int g = KC; g < P.cols; g += 64) {
-            const float x = g + lane < P.cols ? load(g + lane) : __builtin_nanf("");
-            uint64_t m = ballot(x > root);
-            while (m) {
-                const int Ln = __builtin_ctzll(m);
-                hv = wrl_f(hv, rdl_f(x, Ln), 0);
-                hi = wrl_i(hi, g + Ln, 0);
-                heap_sift(hv, hi, 0, KC);
-                root = rdl_f(hv, 0);
-                m = ballot(x > root) & (Ln == 63 ? 0ull : (~0ull << (Ln + 1)));
-            }
-        }
-        for (int a = 0; a < KC; ++a) {
+        auto top = [&]() {
+            const float r = rdl_f(hv, 0);
+            return r == r ? f32_key(r) : 0xFFFFFFFFu;
+        };
+        replay(top(), [&](uint32_t k, int32_t id) {
+            hv = wrl_f(hv, key_f32(k), 0);
+            hi = wrl_i(hi, id, 0);
+            heap_sift(hv, hi, 0, KC);
+            return top();
+        });
+        for (int a = 0; a < KC; ++a) {                      // the selection sort
             int m = a;
             float vm = rdl_f(hv, a);
             for (int b = a + 1; b < KC; ++b) {
@@ -943,73 +980,43 @@ __device__ __forceinline__ void parts_replay(const TreeParams& P, const TreeLayo
                 if (vb > vm) { m = b; vm = vb; }
             }
             const int32_t im = rdl_i(hi, m);
-            if (lane == 0) { out_v[a] = vm; out_i[a] = im; }
+            ri = lane == a ? im : ri;
             hv = wrl_f(hv, rdl_f(hv, a), m);
             hi = wrl_i(hi, rdl_i(hi, a), m);
         }
-        return;
-    }
-    uint32_t hk[TK_FAST_K];
-    int32_t hi[TK_FAST_K];
+    } else {
+        uint32_t hk[TK_FAST_K];
+        int32_t hi[TK_FAST_K];
 #pragma unroll
-    for (int i = 0; i < TK_FAST_K; ++i) {
-        hk[i] = i < KC ? (uint32_t)__builtin_amdgcn_readlane((int)f32_key(f0), i) : 0u;
-        hi[i] = i;
-    }
-    uheap_build<KC, KC / 2 - 1>(hk, hi);
-    uint32_t root = hk[0];
-    // One copy of the replay: the code runs once per row, so its length is
-    // instruction fetch (unrolled over the parts it took 113 us).
-#pragma unroll 1
-    for (int p = 0; p < P.parts; ++p) {
-        if (p % TK_PSTAGE == 0) fetch(p);
-        const uint32_t stored = (uint32_t)__builtin_amdgcn_readlane((int)pn, p);
-        const bool raw = stored > TK_PSLOTS - 1;            // not all stored: the part's values
-        const int base = p * TK_PART;
-        const int n = !raw ? (int)stored : P.cols - base < TK_PART ? P.cols - base : TK_PART;
-#pragma unroll 1
-        for (int g = 0; g < n; g += 64) {                   // 64 values in id order (key 0: none)
-            const int e = g + lane;
-            uint32_t x = 0u;
-            int32_t xj = base + e;
-            if (raw) {
-                const float f = e < n ? load(base + e) : __builtin_nanf("");
-                x = xj >= KC && f == f ? f32_key(f) : 0u;
-            } else {
-                const uint64_t v = g == 0 ? stage[p % TK_PSTAGE][lane]
-                                          : slots[(size_t)p * TK_PSLOTS + 1 + (e < n ? e : g)];
-                x = e < n ? (uint32_t)(v >> 32) : 0u;
-                xj = (int32_t)(uint32_t)v;
-            }
-            uint64_t m = ballot(x > root);
-            while (m) {
-                const int Ln = __builtin_ctzll(m);
-                hk[0] = (uint32_t)__builtin_amdgcn_readlane((int)x, Ln);
-                hi[0] = __builtin_amdgcn_readlane(xj, Ln);
-                uheap_sift<KC, 0>(hk, hi);
-                root = hk[0];
-                m = ballot(x > root) & (Ln == 63 ? 0ull : (~0ull << (Ln + 1)));
-            }
+        for (int i = 0; i < TK_FAST_K; ++i) {
+            hk[i] = i < KC ? (uint32_t)__builtin_amdgcn_readlane((int)f32_key(f0), i) : 0u;
+            hi[i] = i;
         }
-    }
-    int32_t ri = 0;
+        uheap_build<KC, KC / 2 - 1>(hk, hi);
+        replay(hk[0], [&](uint32_t k, int32_t id) {
+            hk[0] = k;
+            hi[0] = id;
+            uheap_sift<KC, 0>(hk, hi);
+            return hk[0];
+        });
 #pragma unroll
-    for (int a = 0; a < KC; ++a) {                          // the selection sort over the slots
-        uint32_t vm = hk[a];
-        int32_t im = hi[a];
-        int m = a;
+        for (int a = 0; a < KC; ++a) {                      // the selection sort over the slots
+            uint32_t vm = hk[a];
+            int32_t im = hi[a];
+            int m = a;
 #pragma unroll
-        for (int b = a + 1; b < KC; ++b) {
-            const bool gt = hk[b] > vm;
-            vm = gt ? hk[b] : vm;
-            im = gt ? hi[b] : im;
-            m = gt ? b : m;
-        }
-        ri = lane == a ? im : ri;
+            for (int b = a + 1; b < KC; ++b) {
+                const bool gt = hk[b] > vm;
+                vm = gt ? hk[b] : vm;
+                im = gt ? hi[b] : im;
+                m = gt ? b : m;
+            }
+            ri = lane == a ? im : ri;
 #pragma unroll
-        for (int b = a + 1; b < KC; ++b) {
-            hk[b] = m == b ? hk[a] : hk[b];
-            hi[b] = m == b ? hi[a] : hi[b];
+            for (int b = a + 1; b < KC; ++b) {
+                hk[b] = m == b ? hk[a] : hk[b];
+                hi[b] = m == b ? hi[a] : hi[b];
+            }
         }
     }
     if (lane < KC) {

@@ -219,3 +219,26 @@ def test_eagle3_tree_state_sizes(gpu, oracle):
         # rows are not split in the smaller states: the candidate slots stay as they were
         end = off + (split if nb == split and off == 0 else small)
         assert bool((buf[end:] == 0xAB).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_eagle3_split_rows_nan_heaps(gpu, oracle, dtype):
+    """NaNs at any places of the first k values, which fix parts of the heap,
+    with ties and more NaNs behind them: the candidates of the parts hold every
+    value that the reference's float compares let in."""
+    import torch
+    import llima_amd
+    rng = np.random.default_rng(12)
+    for k, cols in [(2, 4097), (3, 9000), (5, 32000), (7, 4096), (8, 12289), (11, 9000), (16, 8193)]:
+        tree = llima_amd.Eagle3DraftTree(torch.zeros(cols, dtype=torch.int32, device=gpu), topk=k,
+                                         depth=1)
+        masks = [1 << i for i in range(k)] + [int(m) for m in rng.integers(1, 1 << k, 12)] + [(1 << k) - 1]
+        for m in masks:
+            _say("eagle3 nan heap", dtype, k, cols, bin(m))
+            x = (rng.normal(0, 3, cols) if m & 1 else rng.integers(-9, 10, cols)).astype(np.float32)
+            if m % 3 == 0:
+                x = np.sort(x)                             # more candidates than a part stores
+            x[:k][[(m >> i) & 1 == 1 for i in range(k)]] = np.nan
+            x[k::11] = np.nan
+            xb = wl.f32_to_bf16_bits(x) if dtype == "bf16" else x
+            assert (_np(tree.begin(_t(xb, gpu))) == oracle.topk(xb[None], k)[0][0]).all()
