@@ -340,16 +340,16 @@ __device__ __forceinline__ void topk_row_generic(const TL* rowp, int cols, int k
 // sift-down step is a few register moves and compares instead of readlane
 // round trips.  Keys compare as the floats do (order-preserving, -0 folded
 // onto +0; no NaN is ever in the heap on this path).  Each thread's k-th
-// largest key comes from a sorted list of its TK_FAST_K largest (one max/min
-// pair per list entry and value).
-#define TK_FAST_K 16                      // keys a register heap holds at most
+// largest key comes from a sorted list of its k largest (one max/min pair per
+// list entry and value).  k from 9 on takes the generic heap here: the rows of
+// a draft tree, whose k may be larger, are split into parts (further down).
 #define TK_VPT 16
 #define TK_FTILE (TK_WG * TK_VPT)
 
 // Sift-down from slot NODE of a heap of KC keys: indices are compile-time
 // constants, so the heap stays in registers.
 template <int KC, int NODE>
-__device__ __forceinline__ void uheap_sift(uint32_t (&hk)[TK_FAST_K], int32_t (&hi)[TK_FAST_K]) {
+__device__ __forceinline__ void uheap_sift(uint32_t (&hk)[KC], int32_t (&hi)[KC]) {
     constexpr int C = 2 * NODE + 1;
     if constexpr (C < KC) {
         bool right = false;
@@ -376,7 +376,7 @@ __device__ __forceinline__ void uheap_sift(uint32_t (&hk)[TK_FAST_K], int32_t (&
 
 // The reference's heapify of the first KC values: sift-down from KC/2 - 1 to 0.
 template <int KC, int J>
-__device__ __forceinline__ void uheap_build(uint32_t (&hk)[TK_FAST_K], int32_t (&hi)[TK_FAST_K]) {
+__device__ __forceinline__ void uheap_build(uint32_t (&hk)[KC], int32_t (&hi)[KC]) {
     if constexpr (J >= 0) {
         uheap_sift<KC, J>(hk, hi);
         uheap_build<KC, J - 1>(hk, hi);
@@ -432,7 +432,7 @@ __device__ __forceinline__ void tk_keys(const llima_u32x4 (&q)[TK_VPT * sizeof(T
 
 // v into the descending list L[0, KC) of the KC largest keys (with multiplicity).
 template <int KC>
-__device__ __forceinline__ void tk_list_put(uint32_t (&L)[TK_FAST_K], uint32_t v) {
+__device__ __forceinline__ void tk_list_put(uint32_t (&L)[KC], uint32_t v) {
 #pragma unroll
     for (int i = KC - 1; i > 0; --i) {
         const uint32_t lo = L[i - 1] < v ? L[i - 1] : v;
@@ -452,10 +452,10 @@ __device__ __forceinline__ void topk_row_fast(const TL* rowp, int cols, bool vec
     constexpr int k = KC;
     constexpr int NQ = TK_VPT * (int)sizeof(TL) / 16;
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
-    uint32_t hk[TK_FAST_K];                // wavefront 0: the heap, every lane alike
-    int32_t hi[TK_FAST_K];
+    uint32_t hk[KC];                // wavefront 0: the heap, every lane alike
+    int32_t hi[KC];
 #pragma unroll
-    for (int i = 0; i < TK_FAST_K; ++i) { hk[i] = 0u; hi[i] = 0; }
+    for (int i = 0; i < KC; ++i) { hk[i] = 0u; hi[i] = 0; }
     uint32_t carry = 0u;                   // the heap root after the earlier tiles
     for (int base = 0; base < cols; base += TK_FTILE) {
         const int ib = base + t * TK_VPT;
@@ -464,10 +464,10 @@ __device__ __forceinline__ void topk_row_fast(const TL* rowp, int cols, bool vec
         // ---- the block's k-th largest key, the bound from the earlier blocks
         uint32_t kth;
         {
-            uint32_t kk[TK_VPT], L[TK_FAST_K];
+            uint32_t kk[TK_VPT], L[KC];
             tk_keys<TL>(q, kk);
 #pragma unroll
-            for (int i = 0; i < TK_FAST_K; ++i) L[i] = 0u;
+            for (int i = 0; i < KC; ++i) L[i] = 0u;
 #pragma unroll
             for (int e = 0; e < TK_VPT; ++e) tk_list_put<KC>(L, kk[e]);
             kth = L[k - 1];
@@ -482,10 +482,10 @@ __device__ __forceinline__ void topk_row_fast(const TL* rowp, int cols, bool vec
         // ---- candidates: above the bound and the block's own running k-th key
         uint32_t cmask = 0;
         {
-            uint32_t kk[TK_VPT], L[TK_FAST_K];
+            uint32_t kk[TK_VPT], L[KC];
             tk_keys<TL>(q, kk);
 #pragma unroll
-            for (int i = 0; i < TK_FAST_K; ++i) L[i] = 0u;
+            for (int i = 0; i < KC; ++i) L[i] = 0u;
 #pragma unroll
             for (int e = 0; e < TK_VPT; ++e) {
                 const uint32_t thr = L[k - 1] > bound ? L[k - 1] : bound;
@@ -500,8 +500,7 @@ __device__ __forceinline__ void topk_row_fast(const TL* rowp, int cols, bool vec
             uint32_t kk[TK_VPT];
             tk_keys<TL>(q, kk);
 #pragma unroll
-            for (int e = 0; e < TK_FAST_K; ++e)
-                if (e < k) sh.init_k[e] = kk[e];
+            for (int e = 0; e < k; ++e) sh.init_k[e] = kk[e];
         }
         __syncthreads();
         uint32_t off = ci - cnt, total = 0;
@@ -693,7 +692,7 @@ __device__ __forceinline__ void logsoftmax_rows(const float* v, int rows, int n,
     for (int q = t; q < rows * n; q += (int)blockDim.x) out[q] = v[q] - shift[q / n];
 }
 
-// topk<float> (the reference's heap) of n values in LDS, k = KC <= TK_FAST_K,
+// topk<float> (the reference's heap) of n values in LDS, k = KC,
 // by wavefront 0 (every lane alike) with the heap in scalar registers: the
 // first KC values heapified, then every value above the root in index order
 // (a ballot per 64 values finds them), then the selection sort.  Returns false
@@ -702,19 +701,15 @@ __device__ __forceinline__ void logsoftmax_rows(const float* v, int rows, int n,
 template <int KC>
 __device__ __forceinline__ bool heap_small(const float* x, int n, int32_t* out_i, float* out_v) {
     const int lane = (int)lane_id();
-    uint32_t hk[TK_FAST_K];
-    int32_t hi[TK_FAST_K];
+    uint32_t hk[KC];
+    int32_t hi[KC];
     bool nan0 = false;
 #pragma unroll
-    for (int i = 0; i < TK_FAST_K; ++i) {
-        hk[i] = 0u;
-        hi[i] = 0;
-        if (i < KC) {
-            const float f = x[i];
-            nan0 = nan0 || f != f;
-            hk[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)f32_key(f));
-            hi[i] = i;
-        }
+    for (int i = 0; i < KC; ++i) {
+        const float f = x[i];
+        nan0 = nan0 || f != f;
+        hk[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)f32_key(f));
+        hi[i] = i;
     }
     if (nan0) return false;
     uheap_build<KC, KC / 2 - 1>(hk, hi);
@@ -761,8 +756,8 @@ __device__ __forceinline__ bool heap_small(const float* x, int n, int32_t* out_i
     return true;
 }
 
-// heap_small for a run-time k (wavefront 0); false when k > TK_FAST_K or a
-// NaN is among the first k values.
+// heap_small for a run-time k (wavefront 0); false when k > 8 or a NaN is
+// among the first k values.
 __device__ __forceinline__ bool heap_small_k(const float* x, int n, int k, int32_t* out_i,
                                              float* out_v) {
     switch (k) {
@@ -823,10 +818,10 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
     const int ib = part * TK_PART + t * TK_VPT;
     llima_u32x4 q[NQ];
     tk_raw<TL>(rowp, ib, P.cols, P.vec != 0, q);
-    uint32_t kk[TK_VPT], Lk[TK_FAST_K];
+    uint32_t kk[TK_VPT], Lk[KC];
     tk_keys<TL>(q, kk);
 #pragma unroll
-    for (int i = 0; i < TK_FAST_K; ++i) Lk[i] = 0u;
+    for (int i = 0; i < KC; ++i) Lk[i] = 0u;
 #pragma unroll
     for (int e = 0; e < TK_VPT; ++e) tk_list_put<KC>(Lk, kk[e]);
     // the KC largest keys of all earlier threads: a scan over the lanes, then
@@ -865,7 +860,7 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
     // a value enters when it exceeds the k-th largest before it (ids below k
     // start the heap and are not written)
 #pragma unroll
-    for (int i = 0; i < TK_FAST_K; ++i) Lk[i] = i < N ? A[i < N ? i : 0] : 0u;
+    for (int i = 0; i < KC; ++i) Lk[i] = A[i];
     uint32_t cmask = 0;
 #pragma unroll
     for (int e = 0; e < TK_VPT; ++e) {
@@ -985,11 +980,11 @@ __device__ __forceinline__ void parts_replay(const TreeParams& P, const TreeLayo
             hi = wrl_i(hi, rdl_i(hi, a), m);
         }
     } else {
-        uint32_t hk[TK_FAST_K];
-        int32_t hi[TK_FAST_K];
+        uint32_t hk[KC];
+        int32_t hi[KC];
 #pragma unroll
-        for (int i = 0; i < TK_FAST_K; ++i) {
-            hk[i] = i < KC ? (uint32_t)__builtin_amdgcn_readlane((int)f32_key(f0), i) : 0u;
+        for (int i = 0; i < KC; ++i) {
+            hk[i] = (uint32_t)__builtin_amdgcn_readlane((int)f32_key(f0), i);
             hi[i] = i;
         }
         uheap_build<KC, KC / 2 - 1>(hk, hi);
