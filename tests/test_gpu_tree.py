@@ -76,14 +76,17 @@ def test_topk_strided_rows(gpu, oracle):
     assert (_np(idx) == oracle.topk(np.ascontiguousarray(x[:, 1:5000]), 5)[0]).all()
 
 
-def _run_tree(gpu, oracle, root, levels, d2t, K, depth, total, sample):
+def _run_tree(gpu, oracle, root, levels, d2t, K, depth, total, sample, pad=0):
     import llima_amd
     tree = llima_amd.Eagle3DraftTree(_t(d2t, gpu), topk=K, depth=depth)
     e = oracle.eagle3_tree(root, levels, d2t, K, depth, total, sample, cr=True)
     ids = tree.begin(_t(root, gpu))
     assert (_np(ids) == e["inputs"][0]).all()
     for lv in range(1, depth):
-        ids, prow, mask = tree.grow(_t(levels[lv - 1], gpu))
+        rows = levels[lv - 1]
+        if pad:                                          # a slice of wider rows
+            rows = np.concatenate([rows, np.full((K, pad), rows.max(), rows.dtype)], axis=1)
+        ids, prow, mask = tree.grow(_t(rows, gpu)[:, :levels.shape[2]])
         assert (_np(ids) == e["inputs"][lv]).all(), lv
         assert (_np(prow) == e["parent_rows"][lv - 1]).all(), lv
         assert (_np(mask) == e["masks"][lv - 1][:, :K * (lv + 1)]).all(), lv
@@ -242,3 +245,29 @@ def test_eagle3_split_rows_nan_heaps(gpu, oracle, dtype):
             x[k::11] = np.nan
             xb = wl.f32_to_bf16_bits(x) if dtype == "bf16" else x
             assert (_np(tree.begin(_t(xb, gpu))) == oracle.topk(xb[None], k)[0][0]).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("K,Vd,pad", [(5, 9001, 0), (5, 12288, 7), (10, 8200, 8), (16, 4160, 3), (16, 9000, 0)])
+def test_eagle3_split_rows_mixed_levels(gpu, oracle, dtype, K, Vd, pad):
+    """Levels whose rows differ in kind: one ascending (more candidates than a
+    part stores), one with NaNs among its first k, one of infinities, one of
+    ties, one flat, the rest normal, each replayed by a wavefront of its own;
+    with rows wider apart than Vd and not 16-byte aligned."""
+    _say("eagle3 mixed levels", dtype, K, Vd, pad)
+    rng = np.random.default_rng(K * Vd + pad)
+    depth, total = 3, 20
+    root = rng.normal(0, 3, Vd).astype(np.float32)
+    levels = rng.normal(0, 3, (depth - 1, K, Vd)).astype(np.float32)
+    for lv in range(depth - 1):
+        at = rng.permutation(K)[:5]
+        levels[lv, at[0]] = np.sort(levels[lv, at[0]])
+        levels[lv, at[1], rng.integers(0, K, 2)] = np.nan
+        levels[lv, at[2], ::5] = -np.inf
+        levels[lv, at[2], Vd // 2] = np.inf
+        levels[lv, at[3]] = rng.integers(-3, 4, Vd)
+        levels[lv, at[4]] = 0.5
+    if dtype == "bf16":
+        root, levels = wl.f32_to_bf16_bits(root), wl.f32_to_bf16_bits(levels)
+    d2t = rng.integers(0, 1000, Vd).astype(np.int32)
+    _run_tree(gpu, oracle, root, levels, d2t, K, depth, total, 3, pad=pad)
