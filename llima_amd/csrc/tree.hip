@@ -828,7 +828,7 @@ __global__ __launch_bounds__(TREE_WG) void eagle3_parts_kernel(TreeParams P) {
     // the earlier waves' lists
     uint32_t A[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) A[i] = Lk[i];
+    for (int i = 0; i < N; ++i) A[i] = i < KC ? Lk[i < KC ? i : 0] : 0u;
     auto scan_step = [&](auto dpp) {
         uint32_t B[N];
 #pragma unroll
