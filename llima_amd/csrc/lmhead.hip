@@ -244,7 +244,8 @@ __global__ __launch_bounds__(LMH_WG) void lmh_rows(LmhParams P, int b0, int nb) 
 
 // ------------------------------------------------------------------ MFMA path
 // Batches wider than one GEMV pass: gfx950's v_mfma_f32_32x32x16_bf16 tiles,
-// the weight read once per pass of up to 128 (lmh_mfma) or 256 (lmh_tiles) rows.  Lane l supplies row
+// the weight read once for up to 128 rows (lmh_mfma) or in passes of 128 or 256
+// that share the reads (lmh_tiles).  Lane l supplies row
 // (A: a hidden row) or column (B: a vocab row) l % 32 and 8 consecutive values
 // of k; the k assignment only has to be the same for both operands, and step s
 // of a 64-id chunk gives lane half g the ids 16 s + 8 g .. 16 s + 8 g + 7, so
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(LMH_WG) void lmh_rows(LmhParams P, int b0, int nb) 
 // is not the GEMV path's.
 typedef __bf16 lmh_b8 __attribute__((ext_vector_type(8)));
 typedef float lmh_acc __attribute__((ext_vector_type(16)));
-#define LMH_MB 128                     // hidden rows of lmh_mfma's one pass at most
+#define LMH_MB 128                     // hidden rows of lmh_mfma at most
 
 __device__ __forceinline__ uint64_t lmh_key(float s, int n, int V) {
     return s == s && n < V ? ((uint64_t)f32_key(s) << 32) | (uint32_t)~(uint32_t)n : 0ull;
@@ -323,23 +324,23 @@ __device__ __forceinline__ uint64_t lmh_max_u64(uint64_t a, uint64_t b) { return
 __device__ __forceinline__ float lmh_add_f32(float a, float b) { return a + b; }
 
 // The epilogue of one 32 x 32 accumulator tile over WR column blocks: lane
-// (r, g) holds v[i][j], the logit of tile row i % 4 + 8 (i / 4) + 4 g (pass row
+// (r, g) holds v[i][j], the logit of tile row i % 4 + 8 (i / 4) + 4 g (hidden row
 // mbase + that) and column ncol[j].  Writes the logits (when asked) and each
 // row's greatest key over the wave's 32 WR columns into key slot wv; with SC
 // also the slot's sum of exp(logit - its maximum) and the target's logit (tg[i]:
-// row i's target, -1 for rows past nb).
+// row i's target, -1 for rows past B).
 template <int WR, bool SC>
 __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v)[16][WR],
-                                             const int (&ncol)[WR], int mbase, int b0, int nb,
-                                             int wv, int r, int g, const int32_t (&tg)[16]) {
-    const int V = P.V;
+                                             const int (&ncol)[WR], int mbase, int wv, int r,
+                                             int g, const int32_t (&tg)[16]) {
+    const int B = P.B, V = P.V;
     if (P.out_logits) {                                      // uniform
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int m = mbase + (i & 3) + 8 * (i >> 2) + 4 * g;
 #pragma unroll
             for (int j = 0; j < WR; ++j)
-                if (m < nb && ncol[j] < V) lmh_store_logit(P, (size_t)(b0 + m) * V + ncol[j], v[i][j]);
+                if (m < B && ncol[j] < V) lmh_store_logit(P, (size_t)m * V + ncol[j], v[i][j]);
         }
     }
     uint64_t k[16];
@@ -351,8 +352,8 @@ __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v
     }
     const uint64_t best = half_reduce_scatter16<uint64_t>(k, r, lmh_max_u64);
     const int ir = (r >> 1) & 15, mr = mbase + (ir & 3) + 8 * (ir >> 2) + 4 * g;
-    const bool st = (r & 1) == 0 && mr < nb;                 // one lane per row stores
-    if (st) P.keys[(size_t)(b0 + mr) * P.NW + wv] = best;
+    const bool st = (r & 1) == 0 && mr < B;                  // one lane per row stores
+    if (st) P.keys[(size_t)mr * P.NW + wv] = best;
     if constexpr (SC) {
         uint32_t hv[16];                                     // each row's maximum key
         half_all_gather16((uint32_t)(best >> 32), r, hv);
@@ -369,14 +370,14 @@ __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v
             }
         }
         const float sw = half_reduce_scatter16<float>(e, r, lmh_add_f32);
-        if (st) P.sums[(size_t)(b0 + mr) * P.NW + wv] = sw;
+        if (st) P.sums[(size_t)mr * P.NW + wv] = sw;
         if (hit) {                                           // one lane of the grid per row
 #pragma unroll
             for (int i = 0; i < 16; ++i)
 #pragma unroll
                 for (int j = 0; j < WR; ++j)
                     if (ncol[j] < V && ncol[j] == tg[i])
-                        P.tval[b0 + mbase + (i & 3) + 8 * (i >> 2) + 4 * g] = v[i][j];
+                        P.tval[mbase + (i & 3) + 8 * (i >> 2) + 4 * g] = v[i][j];
         }
     }
 }
@@ -393,10 +394,10 @@ __device__ __forceinline__ void lmh_tile_out(const LmhParams& P, const float (&v
 // are in flight while one feeds the MFMAs: a chunk's loads are requested R
 // iterations before it is staged.
 template <int NWN, int WM, int R, int KC, bool SC>
-__global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, int nb) {
+__global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P) {
     constexpr int NT = 64 * NWN * WM;                        // threads
     constexpr int WR = 32 * NWN;                             // vocab rows of the workgroup
-    constexpr int M = 64 * WM;                               // hidden rows of the pass
+    constexpr int M = 64 * WM;                               // hidden rows of the tile
     constexpr int PPR = KC / 8;                              // 16-byte pieces per row per chunk
     constexpr int LDSR = 2 * KC + 16;                        // bytes per staged row (16-byte aligned)
     constexpr int WQ = WR * PPR / NT;                        // weight pieces per thread per chunk
@@ -407,7 +408,7 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, g = lane >> 5, r = lane & 31;
     const int wn = wave % NWN, wm = wave / NWN;              // vocab tile, hidden group
     const int n0 = (int)blockIdx.x * WR;
-    const int H = P.H, V = P.V, nch = H / KC;
+    const int B = P.B, H = P.H, V = P.V, nch = H / KC;
     // global -> LDS mapping: piece p = t + NT q is row p / PPR, 16-byte column p % PPR
     const int pc = t % PPR;
     const uint16_t* gw[WQ];
@@ -419,8 +420,8 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
     const uint16_t* gx[XQ];
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
-        const int m = (t + NT * q) / PPR;                    // rows past nb read row b0
-        gx[q] = P.hidden + (size_t)(b0 + (m < nb ? m : 0)) * H + pc * 8;
+        const int m = (t + NT * q) / PPR;                    // rows past B read row 0
+        gx[q] = P.hidden + (size_t)(m < B ? m : 0) * H + pc * 8;
     }
     llima_u32x4 rw[R][WQ], rx[R][XQ];
     auto fetch = [&](int c, llima_u32x4 (&fw)[WQ], llima_u32x4 (&fx)[XQ]) {
@@ -476,15 +477,6 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
             __syncthreads();
         }
     }
-    // key slots past this grid's waves (a grid of 128-row tiles can leave up
-    // to 4 of the P.NW slots, counted in 256-row tiles): no logit
-    if (blockIdx.x == gridDim.x - 1) {
-        const int w0 = (int)gridDim.x * NWN, nx = P.NW - w0;
-        for (int e = t; e < nx * nb; e += NT) {
-            P.keys[(size_t)(b0 + e / nx) * P.NW + w0 + e % nx] = 0;
-            if constexpr (SC) P.sums[(size_t)(b0 + e / nx) * P.NW + w0 + e % nx] = 0.0f;
-        }
-    }
     // epilogue: softcap, logits, and per hidden row the greatest key of the wave's 32 columns
     const int wv = (int)blockIdx.x * NWN + wn;
     const int ncol[1] = {n0 + wn * 32 + r};
@@ -494,7 +486,7 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int m = wm * 64 + mt * 32 + (i & 3) + 8 * (i >> 2) + 4 * g;
-            tgv[mt][i] = SC && m < nb ? P.targets[b0 + m] : -1;
+            tgv[mt][i] = SC && m < B ? P.targets[m] : -1;
         }
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
@@ -502,7 +494,7 @@ __global__ __launch_bounds__(64 * NWN * WM) void lmh_mfma(LmhParams P, int b0, i
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i][0] = acc[mt][i];
         lmh_logit_tile<1>(v, P);
-        lmh_tile_out<1, SC>(P, v, ncol, wm * 64 + mt * 32, b0, nb, wv, r, g, tgv[mt]);
+        lmh_tile_out<1, SC>(P, v, ncol, wm * 64 + mt * 32, wv, r, g, tgv[mt]);
     }
 }
 
@@ -1045,7 +1037,7 @@ __global__ void lmh_tree(const int32_t* ids, const float* vals, int K, const int
 // whole rows of the plain one.
 //
 // lmh_packed: 256-thread workgroups; each wave takes WR consecutive row
-// blocks of 32 vocab rows (adjacent in the packed layout) against the pass's
+// blocks of 32 vocab rows (adjacent in the packed layout) against up to
 // 32 NMT hidden rows.  Those are staged in LDS per range of KR ids, once per
 // workgroup, in the same fragment order (1 KB per 16 ids and 32 rows, a
 // 16-byte LDS read per lane), double-buffered with one barrier per range;
@@ -1057,19 +1049,18 @@ __global__ void lmh_tree(const int32_t* ids, const float* vals, int K, const int
 #define LMP_WG 256
 #define LMP_WAVES (LMP_WG / 64)
 #define LMP_SG 8                       // k-steps per contiguous group of a row block
-#define LMP_MB 64                      // hidden rows per pass
+#define LMP_MB 64                      // hidden rows of lmh_packed at most
 #define LMP_HM 256                     // the H multiple of the packed layout
 
 template <int NMT, int WR, int R, int KR, bool SC>
-__global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t* packed, int b0,
-                                                     int nb) {
+__global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t* packed) {
     constexpr int SPR = KR / 16;                             // k-steps per range
     constexpr int XB = SPR * NMT * 1024;                     // bytes of a staged range
     constexpr int XQ = XB / 16 / LMP_WG;                     // 16-byte pieces per thread
     static_assert(XQ * 16 * LMP_WG == XB && SPR % R == 0 && KR % LMP_HM == 0, "even split");
     __shared__ __align__(16) uint8_t lx[2][XB];
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, g = lane >> 5, r = lane & 31;
-    const int H = P.H, V = P.V, NS = H / 16, NRB = (V + 31) / 32, nkr = H / KR;
+    const int B = P.B, H = P.H, V = P.V, NS = H / 16, NRB = (V + 31) / 32, nkr = H / KR;
     const int wv = (int)blockIdx.x * LMP_WAVES + wave;       // key slot
     const int rb0 = wv * WR;                                 // >= NRB: spare row blocks
     const size_t gstride = (size_t)NRB * LMP_SG * 1024;      // bytes between groups
@@ -1083,14 +1074,14 @@ __global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t*
     };
     // staging: piece p = t + LMP_WG q is lane p % 64 of fragment (s, mt) =
     // (p / 64 / NMT, p / 64 % NMT) of the range: 16 bytes of hidden row
-    // 32 mt + p % 32 (rows past nb read row b0; their sums are not used) at ids
+    // 32 mt + p % 32 (rows past B read row 0; their sums are not used) at ids
     // 16 s + 8 (p % 64 / 32) of the range
     const uint16_t* gx[XQ];
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
         const int p = t + LMP_WG * q, fr = p >> 6, mt = fr % NMT, s = fr / NMT;
         const int m = 32 * mt + (p & 31);
-        gx[q] = P.hidden + (size_t)(b0 + (m < nb ? m : 0)) * H + 16 * s + 8 * ((p & 63) >> 5);
+        gx[q] = P.hidden + (size_t)(m < B ? m : 0) * H + 16 * s + 8 * ((p & 63) >> 5);
     }
     llima_u32x4 rx[XQ];
     auto fetch_x = [&](int kr) {
@@ -1139,15 +1130,6 @@ __global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t*
         stage_x((kr + 1) & 1);                               // its last readers passed the last barrier
         __syncthreads();
     }
-    // key slots past this grid's waves (a pass with more row blocks per wave
-    // than another uses fewer of the P.NW slots): no logit, spread over the grid
-    {
-        const int w0 = (int)gridDim.x * LMP_WAVES, nx = P.NW - w0;
-        for (int e = (int)blockIdx.x * LMP_WG + t; e < nx * nb; e += (int)gridDim.x * LMP_WG) {
-            P.keys[(size_t)(b0 + e / nx) * P.NW + w0 + e % nx] = 0;
-            if constexpr (SC) P.sums[(size_t)(b0 + e / nx) * P.NW + w0 + e % nx] = 0.0f;
-        }
-    }
     // epilogue: softcap, logits, per hidden row the greatest key of the wave's
     // 32 WR vocab rows
     int ncol[WR];
@@ -1159,7 +1141,7 @@ __global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t*
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int m = mt * 32 + (i & 3) + 8 * (i >> 2) + 4 * g;
-            tgv[mt][i] = SC && m < nb ? P.targets[b0 + m] : -1;
+            tgv[mt][i] = SC && m < B ? P.targets[m] : -1;
         }
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt) {
@@ -1169,7 +1151,7 @@ __global__ __launch_bounds__(LMP_WG) void lmh_packed(LmhParams P, const uint8_t*
 #pragma unroll
             for (int j = 0; j < WR; ++j) v[i][j] = acc[j][mt][i];
         lmh_logit_tile<WR>(v, P);
-        lmh_tile_out<WR, SC>(P, v, ncol, mt * 32, b0, nb, wv, r, g, tgv[mt]);
+        lmh_tile_out<WR, SC>(P, v, ncol, mt * 32, wv, r, g, tgv[mt]);
     }
 }
 
@@ -1208,11 +1190,10 @@ static int lmh_rows_per_pass(int H) {
 
 using namespace llima;
 
-// Key slots per hidden row of lmh_mfma, one per 32 vocab rows, in whole
-// 256-row tiles (a grid of 128-row tiles writes 0 to the up to 4 slots it
-// leaves), and of lmh_tiles, one per 64.
+// Key slots per hidden row of lmh_mfma, one per 32 vocab rows in whole 128-row
+// tiles, and of lmh_tiles, one per 64.
 static int lmh_mfma_waves(int V) {
-    return (V + 255) / 256 * 8;
+    return (V + 127) / 128 * 4;
 }
 
 static int lmh_tile_slots(int V) {
@@ -1293,8 +1274,8 @@ static int lmh_run_plain(LmhParams& P, hipStream_t st) {
         } else {
             P.NW = lmh_mfma_waves(V);
             const dim3 g128((uint32_t)((V + 127) / 128));
-            if (B <= 64) hipLaunchKernelGGL((lmh_mfma<4, 1, 4, LMH_KC, SC>), g128, dim3(256), 0, st, P, 0, B);
-            else hipLaunchKernelGGL((lmh_mfma<4, 2, 2, LMH_KC, SC>), g128, dim3(512), 0, st, P, 0, B);
+            if (B <= 64) hipLaunchKernelGGL((lmh_mfma<4, 1, 4, LMH_KC, SC>), g128, dim3(256), 0, st, P);
+            else hipLaunchKernelGGL((lmh_mfma<4, 2, 2, LMH_KC, SC>), g128, dim3(512), 0, st, P);
         }
     } else {
         P.NW = lmh_waves(V);
@@ -1491,18 +1472,18 @@ extern "C" int llima_lm_head_score(const void* hidden, const void* weight, int32
     return lmh_run_plain<true>(P, (hipStream_t)stream);
 }
 
-// Row blocks per wave, and ring depth, of lmh_packed passes of 32 and of 64
-// hidden rows.
-#define LMP_WR1 2
+// Row blocks per wave of lmh_packed, and its ring depth for up to 32 and up to
+// 64 hidden rows.
+#define LMP_WR 2
 #define LMP_R1 8
-#define LMP_WR2 2
 #define LMP_R2 4
 #define LMP_KR 256                     // hidden ids per LDS-staged range
 
-// Workgroups of lmh_packed for WR row blocks per wave; its key slots per
-// hidden row are one per wave.
-static int lmp_groups(int V, int wr) {
-    return ((V + 31) / 32 + LMP_WAVES * wr - 1) / (LMP_WAVES * wr);
+// Workgroups of lmh_packed; its key slots per hidden row, one per wave, are as
+// many as lmh_tiles has.
+static_assert(32 * LMP_WR == LMH_SLOT && LMP_WAVES * LMH_SLOT == LMH_NV, "one slot count");
+static int lmp_groups(int V) {
+    return (V + LMH_NV - 1) / LMH_NV;
 }
 
 extern "C" size_t llima_lm_head_packed_bytes(int32_t V, int32_t H) {
@@ -1510,20 +1491,14 @@ extern "C" size_t llima_lm_head_packed_bytes(int32_t V, int32_t H) {
     return (size_t)((V + 31) / 32) * 32 * (size_t)H * 2;
 }
 
-static int lmp_slots(int V) {
-    const int g1 = lmp_groups(V, LMP_WR1), g2 = lmp_groups(V, LMP_WR2);
-    const int n = (g1 > g2 ? g1 : g2) * LMP_WAVES;
-    return n > lmh_tile_slots(V) ? n : lmh_tile_slots(V);
-}
-
 extern "C" size_t llima_lm_head_argmax_packed_workspace_bytes(int32_t B, int32_t H, int32_t V) {
     if (B <= 0 || llima_lm_head_packed_bytes(V, H) == 0) return 0;
-    return lmh_ws_bytes(B, lmp_slots(V), false);
+    return lmh_ws_bytes(B, lmh_tile_slots(V), false);
 }
 
 extern "C" size_t llima_lm_head_score_packed_workspace_bytes(int32_t B, int32_t H, int32_t V) {
     if (B <= 0 || llima_lm_head_packed_bytes(V, H) == 0) return 0;
-    return lmh_ws_bytes(B, lmp_slots(V), true);
+    return lmh_ws_bytes(B, lmh_tile_slots(V), true);
 }
 
 extern "C" int llima_lm_head_pack(const void* weight, int32_t V, int32_t H, void* packed,
@@ -1542,9 +1517,9 @@ extern "C" int llima_lm_head_pack(const void* weight, int32_t V, int32_t H, void
 // The passes over a packed weight and the finish (lmh_score_finish with SC).
 template <bool SC>
 static int lmh_run_packed(LmhParams& P, const uint8_t* packed, hipStream_t st) {
-    const int B = P.B, V = P.V;
-    const int ng1 = lmp_groups(V, LMP_WR1), ng2 = lmp_groups(V, LMP_WR2);
-    P.NW = lmp_slots(V);
+    const int B = P.B;
+    const dim3 g((uint32_t)lmp_groups(P.V));
+    P.NW = lmh_tile_slots(P.V);
     // Up to 64 rows a wave streams its own vocab rows into registers (165 us at
     // B = 64, H = 4096, V = 128256); above, where that kernel would read the
     // weight again per 64 rows (B = 128 324 us, B = 256 646, B = 512 1287),
@@ -1552,11 +1527,9 @@ static int lmh_run_packed(LmhParams& P, const uint8_t* packed, hipStream_t st) {
     if (B > LMP_MB)
         lmh_run_tiles<true, SC>(P, packed, st);
     else if (B <= 32)
-        hipLaunchKernelGGL((lmh_packed<1, LMP_WR1, LMP_R1, LMP_KR, SC>), dim3(ng1), dim3(LMP_WG), 0,
-                           st, P, packed, 0, B);
+        hipLaunchKernelGGL((lmh_packed<1, LMP_WR, LMP_R1, LMP_KR, SC>), g, dim3(LMP_WG), 0, st, P, packed);
     else
-        hipLaunchKernelGGL((lmh_packed<2, LMP_WR2, LMP_R2, LMP_KR, SC>), dim3(ng2), dim3(LMP_WG), 0,
-                           st, P, packed, 0, B);
+        hipLaunchKernelGGL((lmh_packed<2, LMP_WR, LMP_R2, LMP_KR, SC>), g, dim3(LMP_WG), 0, st, P, packed);
     if (SC) hipLaunchKernelGGL(lmh_score_finish, dim3((uint32_t)B), dim3(LLIMA_WG), 0, st, P);
     else hipLaunchKernelGGL(lmh_finish, dim3((uint32_t)B), dim3(LLIMA_WG), 0, st, P);
     return hipGetLastError() == hipSuccess ? LLIMA_OK : LLIMA_E_HIP;
@@ -1613,7 +1586,7 @@ extern "C" int llima_lm_head_score_packed(const void* hidden, const void* packed
     P.targets = targets;
     P.out_logprob = out_logprob;
     P.out_greedy = out_is_greedy;
-    lmh_ws_split(P, workspace, lmp_slots(V));
+    lmh_ws_split(P, workspace, lmh_tile_slots(V));
     return lmh_run_packed<true>(P, (const uint8_t*)packed, (hipStream_t)stream);
 }
 
