@@ -1362,8 +1362,8 @@ def test_lm_head_bf16_logits_out(gpu, B, H, V, packed):
 
 
 # LM head scoring: the (B, H, V, softcap, packed) cases cover the matrix-vector
-# path (B up to 8), the MFMA tiles (wider batches, H > 4096, two 256-row passes)
-# and the packed weight (32- and 64-row passes, two passes).
+# path (B up to 8), the MFMA tiles (wider batches, H > 4096, three 128-row passes)
+# and the packed weight (up to 32, 64 and 128 rows).
 LM_SCORE_CASES = [(1, 4096, 32768, 0.0, False), (3, 1024, 50000, 30.0, False),
                   (8, 2048, 20000, 0.0, False), (17, 256, 777, 0.0, False),
                   (64, 4096, 20000, 30.0, False), (300, 256, 3001, 0.0, False),
