@@ -314,7 +314,8 @@ int llima_mtp_masked_argmax(const uint16_t* centroid_logits, int64_t centroid_st
  * with LLIMA_LOGITS_OUT_BF16) every logit.  H % 8 == 0, and H <= 4096 unless H % 64 == 0 (then H <= 65536).  The
  * weights are read once per 8 hidden rows (H <= 2048) or 4 (H <= 4096); wider
  * batches, and rows wider than 4096, use MFMA tiles (H % 64 == 0) that read them
- * once for up to 128 rows, and in passes of 256 rows that share the reads above. */
+ * once for up to 128 rows, and above in passes that share the reads (256 rows,
+ * or 128 where 256 would leave half of the CUs without a tile). */
 size_t llima_lm_head_argmax_workspace_bytes(int32_t B, int32_t V);
 int llima_lm_head_argmax(const void* hidden, const void* weight, int32_t B, int32_t H, int32_t V,
                          float softcap, int32_t logit_dtype, int32_t* out_ids, float* out_vals,
@@ -327,8 +328,8 @@ int llima_lm_head_argmax(const void* hidden, const void* weight, int32_t B, int3
  * rows up to a multiple of 32; for each 128 ids, the row blocks in order).  llima_lm_head_argmax_packed takes the packed
  * weight in place of `weight` and gives the same ids, values and logits as
  * llima_lm_head_argmax's MFMA tiles; it reads the weight once for up to 128
- * hidden rows (up to 64 of them each wave streams contiguous memory), and in
- * passes of 256 rows that share the reads above.  Workspace:
+ * hidden rows (up to 64 of them each wave streams contiguous memory), and above
+ * in the passes of the plain weight.  Workspace:
  * llima_lm_head_argmax_packed_workspace_bytes(B, H, V) (0 for invalid sizes).  No counterpart in the reference,
  * whose LM head runs inside its compiled graph (language_part_base.py:171-180):
  * a weight layout chosen at load time, as such graphs choose theirs. */

@@ -604,9 +604,12 @@ __device__ __forceinline__ int lmh_first_max(const float (&x)[32], int g, float&
 // the same bits.
 //
 // Bound: the matrix cores at B > 128 (B = 512, H = 4096, V = 128256: 538 GFLOP
-// in 432 us, 1.25 PFLOP/s; a library product of 8192^3 reaches 1.42), reading
-// the weight at B <= 128 (1.05 GB in 178 us, 5.9 TB/s).  Before: 696 us (plain)
-// and 1287 us (packed) at B = 512, 324 us (packed) at B = 128.
+// in 427 us, 1.26 PFLOP/s; a library product of 8192^3 reaches 1.42), reading
+// the weight at B <= 128 (1.05 GB in 172 us, 6.1 TB/s).  Before: 696 us (plain)
+// and 1287 us (packed) at B = 512, 324 us (packed) at B = 128.  The last turn of
+// the 256 workgroups is as full as the units make it: 501 units (V = 128256, one
+// pass) are 1.96 turns, 392 (V = 100352) 1.53 and 594 (V = 151936) 2.32, and
+// those read the weight at 5.4 TB/s.
 template <int NM, int WVN, int RW, int RX, bool PK, bool SC>
 __global__ __launch_bounds__(256) void lmh_tiles(LmhParams P, const uint8_t* weight, int npass) {
     constexpr int NV = LMH_NV, WMN = 4 / WVN;                // WMN: waves along the hidden rows
@@ -1266,9 +1269,13 @@ static int lmh_run_plain(LmhParams& P, hipStream_t st) {
     if ((B > lmh_rows_per_pass(H) || H > LMH_MAX_H) && H % LMH_KC == 0) {   // MFMA paths
         // Up to 128 rows one pass of lmh_mfma: there both kernels are bound by
         // reading 128-byte pieces of the plain weight's rows, and lmh_mfma has
-        // more of them in flight (B = 64 212 against 238 us, B = 128 235
-        // against 256, H = 4096, V = 128256).  Above, lmh_tiles (B = 256 294
-        // against 350 us, B = 512 436 against 696).
+        // more of them in flight and smaller tiles.  Measured in turn, B = 128:
+        // H = 4096, V = 128256 234 against 277 us, V = 16000 50 against 62;
+        // lmh_tiles is ahead from 50257 ids on at H = 8192 (V = 128256 379
+        // against 445) and by 10 % at H = 4096, V = 50257 without logits, but
+        // the line goes by the batch alone.  Above 128 rows lmh_tiles
+        // (H = 4096, V = 128256: B = 256 301 against 350 us, B = 512 427
+        // against 696).
         if (B > LMH_MB) {
             lmh_run_tiles<false, SC>(P, (const uint8_t*)P.weight, st);
         } else {

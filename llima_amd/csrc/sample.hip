@@ -3816,10 +3816,12 @@ __global__ __launch_bounds__(LLIMA_WG) void dense_bound(SampleParams P) {
     }
 }
 
-// 28 vector instructions per binned value: constants in scalar registers, no
-// test for the row's end, the penalties or an infinite maximum per value (41
-// with them: 19.0 us for 64 rows of 128256 fp32 values, now 17.4; dense_stats,
-// which no longer counts the finite values, 9.3 -> 7.7).  A workgroup's data
+// 28 vector instructions per binned value of a whole fp32 chunk without
+// penalties: constants in scalar registers, no test per value for the row's end
+// or the penalties (dense_unpack's plain branch; bf16 rows, rows with penalties
+// and the last chunk have them) or for an infinite maximum (41 with them: 19.0 us
+// for 64 rows of 128256 fp32 values, now 17.4; dense_stats, which no longer
+// counts the finite values, 9.3 -> 7.7).  A workgroup's data
 // arrives 2.8 to 8.4 us after the first workgroup starts; then unpacking takes
 // 0.6 us, binning 1.8, the window 0.5 and the staging 1.3.
 template <typename TL>

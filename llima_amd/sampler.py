@@ -465,7 +465,9 @@ def score_logits(logits: torch.Tensor, target):
 
     logits [V] with an int target -> (logprob float, is_greedy bool), raising
     RuntimeError for a target outside the vocabulary as the reference does;
-    logits [B, V] with int targets [B] -> (float64 [B], bool [B]) tensors."""
+    logits [B, V] with int targets [B] -> (float64 [B], bool [B]) tensors, ready
+    in the order of the current stream (the call waits for the targets, not for
+    the scores, and cannot be captured)."""
     single = logits.dim() == 1
     x = _rows2d(logits)
     B, V = x.shape
@@ -582,8 +584,8 @@ class PackedLmHead:
     vocab rows x 16 ids, zero rows up to a multiple of 32, 8 KB groups per 32
     rows and 128 ids), so that each wave streams contiguous memory straight
     into the matrix cores.  `data` is the uint8 device tensor; V and H are the
-    weight's shape.  It is read once per pass: up to 64 hidden rows, up to 128,
-    or 256 of a wider batch."""
+    weight's shape.  It is read once for up to 128 hidden rows; wider batches go
+    in passes of 256 rows (128 over a short vocabulary) that share the reads."""
 
     def __init__(self, data: torch.Tensor, V: int, H: int):
         self.data, self.V, self.H = data, V, H
@@ -667,8 +669,8 @@ def lm_head_score(hidden: torch.Tensor, weight, target, softcap: float = 0.0,
     with int targets [B] -> (float64 [B] log-probabilities, bool [B] greedy
     flags), or hidden [H] with an int target -> (float, bool).  The logits are
     lm_head_argmax's (the same softcap and logit_dtype); weight may be a
-    PackedLmHead.  A target outside the vocabulary raises RuntimeError, as
-    score_logits does."""
+    PackedLmHead.  A target outside the vocabulary raises RuntimeError, and the
+    [B] results are ready in the order of the current stream, as score_logits'."""
     single = hidden.dim() == 1
     x = hidden.reshape(1, -1) if single else hidden
     packed = isinstance(weight, PackedLmHead)
